@@ -224,21 +224,27 @@ CELER_FORCEINLINE_FUNCTION void along_step_charged_track(CoreParamsRef const& pa
 
     // Continuous energy loss
     TrackStatus new_status = status;
-    if (part.eloss_process >= 0 && energy > 0)
+    if (part.eloss_process >= 0)
     {
-        bool const apply_cut = post != params.scalars.boundary_action;
-        double const deposited = alongstep::calc_eloss(
-            pp, part, pid, mat, energy, ps.dedx_range[slot], step, apply_cut, rng);
-        if (deposited > 0)
+        if (energy > 0)
         {
-            ps.energy_deposition[slot] += deposited;
-            energy -= deposited;
+            bool const apply_cut = post != params.scalars.boundary_action;
+            double const deposited = alongstep::calc_eloss(
+                pp, part, pid, mat, energy, ps.dedx_range[slot], step, apply_cut, rng);
+            if (deposited > 0)
+            {
+                ps.energy_deposition[slot] += deposited;
+                energy -= deposited;
 #if CELER_PREC_IS_MIXED
-            if (CELER_UNLIKELY(!(energy >= 0 && energy < HUGE_VAL)))
-                energy = 0;
+                if (CELER_UNLIKELY(!(energy >= 0 && energy < HUGE_VAL)))
+                    energy = 0;
 #endif
-            state.particle.energy[slot] = energy;
+                state.particle.energy[slot] = energy;
+            }
         }
+        // Also a lepton that an interaction left (or made) with no energy,
+        // as 32-bit sampling can: without a process at rest it would go on
+        // choosing interactions and make another one of its kind every step
         if (energy == 0)
         {
             if (!part.has_at_rest)

@@ -110,3 +110,36 @@ def test_mixed_workload_sample_completes(host_loop, tmp):
     assert not summary["hit_iteration_limit"]
     # About 1.4e5 track-steps per primary of 1-100 GeV
     assert summary["track_steps"] > 200 * 5e4
+
+
+@pytest.mark.parametrize("particle,status,post", [(0, 4, "range"), (1, 2, "discrete")])
+def test_lepton_without_energy_ends(host_loop, tmp, particle, status, post):
+    """An electron that an interaction left with exactly no energy is killed
+    by its next along-step (left alive it takes zero-length steps that each
+    make another electron of no energy); a positron goes on to annihilate at
+    rest. The pre-step gives either a step of length 0 that ends in the
+    discrete selection."""
+    prob = write_testem3_problem(tmp)
+    fixture = json.loads(open(os.path.join(ROOT, "tests", "golden",
+                                           "mixed_stall_snapshot.json")).read())["snapshot"]
+    ids = action_ids(prob)
+    snap = dict(fixture, phase="along-charged", particle=particle, status=2, energy=0.0,
+                step=0.0, macro_xs=0.0, mfp=1.0, range=0.0, post=ids["discrete"],
+                along=ids["along"])
+    r = subprocess.run([str(host_loop), str(prob), "--replay", json.dumps(snap), "1", "mixed"],
+                       capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr
+    after = json.loads(r.stdout.strip().splitlines()[-1])
+    assert after["energy"] == 0
+    assert (after["status"], after["post"]) == (status, ids[post])
+
+
+def action_ids(prob):
+    """Action IDs of a problem in their fixed order: the physics actions
+    first (discrete and range among them), then the along-step."""
+    from tests import oracle_bind as ob
+
+    labels = ob.Problem(json.loads(open(prob).read())).action_labels()
+    return {"discrete": labels.index("physics-discrete-select"),
+            "range": labels.index("eloss-range"),
+            "along": labels.index("along-step-general-linear")}
