@@ -191,9 +191,14 @@ __global__ void __launch_bounds__(block_size)
 //---------------------------------------------------------------------------//
 // TRACK INITIALIZATION
 //---------------------------------------------------------------------------//
-__global__ void init_prepare_kernel(CoreCounters* c, size_type num_slots)
+__global__ void
+init_prepare_kernel(CoreCounters* c, size_type num_slots, size_type capacity)
 {
-    size_type const n = min(c->num_vacancies, c->num_initializers);
+    // After an overflow the top of the stack was never written: no tracks
+    // start from it in the steps that run until the host sees the error
+    size_type const n = c->num_initializers <= capacity
+                            ? min(c->num_vacancies, c->num_initializers)
+                            : 0;
     c->num_new_tracks = n;
     c->init_base = c->num_initializers;
     c->vacancy_base = c->num_vacancies;
@@ -632,7 +637,7 @@ hipError_t launch_initialize_tracks(CoreParamsRef const& params,
                                     hipStream_t stream)
 {
     unsigned int const nb = num_blocks(state.size);
-    init_prepare_kernel<<<1, 1, 0, stream>>>(state.counters, state.size);
+    init_prepare_kernel<<<1, 1, 0, stream>>>(state.counters, state.size, state.init.capacity);
     if (params.scalars.track_order == TrackOrder::init_charge)
     {
         partition_count_kernel<<<nb, block_size, 0, stream>>>(params, state);
