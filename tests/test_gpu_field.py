@@ -99,3 +99,31 @@ def test_random_tracks_match_oracle(amd, params, oproblem):
             mismatched += 1
             print(f"track {i}: device {dev[i, :, :3].tolist()} oracle {ora[:, :3].tolist()}")
     assert mismatched == 0
+
+
+@pytest.mark.parametrize("ntracks", [1, 3, 64, 65])
+def test_long_chord_searches_match_oracle(amd, params, oproblem, ntracks):
+    """Steps far beyond the helix radius, as tracks in vacuum ask for: the
+    lanes of a wave share the start of the chord search. Waves of one lane,
+    a few, all 64 and one more; every track its own momentum, field and
+    request, among them requests that need no search, directions along the
+    field (accepted at any length) and a second request that starts with
+    the first's chord memory."""
+    rng = np.random.default_rng(ntracks)
+    tracks, steps = [], []
+    for i in range(ntracks):
+        mu = [1.0, -1.0, 0.0][i % 3] if i % 7 == 0 else rng.uniform(-1, 1)
+        phi = rng.uniform(0, 2 * math.pi)
+        st = math.sqrt(1 - mu * mu)
+        d = [st * math.cos(phi), st * math.sin(phi), mu]
+        mom = fc.momentum(10 ** rng.uniform(-2, 4))
+        tracks.append(list(rng.uniform(-4, 4, 3)) + d
+                      + [mom, [-1, 1][i % 2], 0, 0, 10 ** rng.uniform(-1, 1)])
+        steps.append([[2.4e22, 1e8, 3e5, 1e-3, 7.0][i % 5], 1e22, -1, 1e12])
+    dev = amd.verify_field_propagate(params, np.array(tracks), np.array(steps), 0)
+    for t, s, got in zip(tracks, steps, dev):
+        ora = ob.field_propagate(oproblem, t[:3], t[3:6], t[6], t[7], t[8:], s, 0)
+        np.testing.assert_array_equal(got[:, 1:3], ora[:, 1:3])
+        np.testing.assert_array_equal(got[:, 9], ora[:, 9])
+        np.testing.assert_allclose(got[:, 0], ora[:, 0], rtol=1e-10, atol=1e-15)
+        np.testing.assert_allclose(got[:, 3:9], ora[:, 3:9], rtol=1e-10, atol=1e-10)
