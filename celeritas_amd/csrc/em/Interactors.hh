@@ -40,7 +40,7 @@ CELER_FUNCTION std::uint32_t sample_element(PhysicsParamsRef const& p,
                                             ProcessRecord const& proc,
                                             std::uint32_t model_index,
                                             std::uint32_t mat,
-                                            double energy,
+                                            phys::GridPoint& gp,
                                             Engine& rng)
 {
     if (p.num_materials == 0 || p.materials == nullptr)
@@ -58,7 +58,7 @@ CELER_FUNCTION std::uint32_t sample_element(PhysicsParamsRef const& p,
     std::uint32_t i = 0;
     for (; i + 1 < m.num_elements; ++i)
     {
-        if (phys::calc_grid(p.grids[first + i], p.grid_reals, energy) > u)
+        if (phys::calc_grid(p.grids[first + i], p.grid_reals, gp) > u)
             break;
     }
     return i;

@@ -67,7 +67,7 @@ CELER_FORCEINLINE_FUNCTION void along_step_charged_track(CoreParamsRef const& pa
                            ps.dedx_range[slot], 0};
     if (msc_applies)
     {
-        mt.lambda = mt.calc_msc_mfp(energy);
+        mt.lambda = mt.calc_msc_mfp(mt.pre_step());
         if (step <= alongstep::msc_limit_min_fix)
         {
             true_path = step;
@@ -229,8 +229,9 @@ CELER_FORCEINLINE_FUNCTION void along_step_charged_track(CoreParamsRef const& pa
         if (energy > 0)
         {
             bool const apply_cut = post != params.scalars.boundary_action;
+            phys::GridPoint gp = mt.pre_step();
             double const deposited = alongstep::calc_eloss(
-                pp, part, pid, mat, energy, ps.dedx_range[slot], step, apply_cut, rng);
+                pp, part, pid, mat, gp, ps.dedx_range[slot], step, apply_cut, rng);
             if (deposited > 0)
             {
                 ps.energy_deposition[slot] += deposited;

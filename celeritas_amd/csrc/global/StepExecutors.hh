@@ -91,7 +91,8 @@ CELER_FUNCTION void pre_step_track(CoreParamsRef const& params,
     std::uint32_t const mat = material_of(params, state, slot);
     double const energy = state.particle.energy[slot];
     double total = 0;
-    // One log and grid bracket of the energy, shared by the processes
+    // One log and grid bracket of the energy, shared by the processes and
+    // the range
     phys::GridPoint gp(energy);
     for (std::uint32_t i = 0; i < part.num_processes; ++i)
     {
@@ -114,7 +115,7 @@ CELER_FUNCTION void pre_step_track(CoreParamsRef const& params,
         if (part.eloss_process >= 0)
         {
             double const range
-                = phys::calc_range(pp.grids[part.range_grid + mat], pp.grid_reals, energy);
+                = phys::calc_range(pp.grids[part.range_grid + mat], pp.grid_reals, gp);
             ps.dedx_range[slot] = range;
             double const eloss_step = phys::range_to_step(pp.scalars, range);
             if (eloss_step <= step)
@@ -236,9 +237,10 @@ CELER_FUNCTION void discrete_select_track(CoreParamsRef const& params,
     ProcessRecord const& proc = part.process[pidx];
     std::uint8_t action;
     bool rejected = false;
+    phys::GridPoint gp(energy);
     if (proc.integral)
     {
-        double const xs = phys::calc_xs(pp, proc, mat, energy);
+        double const xs = phys::calc_xs(pp, proc, mat, gp);
         if (draw_canonical(rng) * state.phys.per_process_xs[pidx * state.size + slot] > xs)
         {
             rejected = true;
@@ -257,7 +259,7 @@ CELER_FUNCTION void discrete_select_track(CoreParamsRef const& params,
                 mi = k;
         }
         state.phys.element[slot]
-            = static_cast<std::uint8_t>(sample_element(pp, proc, mi, mat, energy, rng));
+            = static_cast<std::uint8_t>(sample_element(pp, proc, mi, mat, gp, rng));
         action = static_cast<std::uint8_t>(proc.models[mi].action);
     }
     rng.store(state.rng, slot);

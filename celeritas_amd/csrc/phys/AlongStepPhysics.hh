@@ -225,16 +225,17 @@ CELER_FUNCTION double calc_eloss(PhysicsParamsRef const& p,
                                  ParticlePhysics const& part,
                                  std::uint32_t pid,
                                  std::uint32_t mat,
-                                 double energy,
+                                 phys::GridPoint& gp,
                                  double range,
                                  double step,
                                  bool apply_cut,
                                  Engine& rng)
 {
+    double const energy = gp.energy;
     double const lowest = p.scalars.lowest_electron_energy;
     if (apply_cut && energy < lowest)
         return energy;
-    double eloss = phys::calc_mean_eloss(p, part, mat, energy, range, step);
+    double eloss = phys::calc_mean_eloss(p, part, mat, gp, range, step);
     if (p.fluct_enabled && eloss < energy)
     {
         // EnergyLossHelper: e+- always use the Urban model above 10 eV
@@ -273,6 +274,21 @@ CELER_FUNCTION double calc_eloss(PhysicsParamsRef const& p,
     return eloss;
 }
 
+template<class Engine>
+CELER_FUNCTION double calc_eloss(PhysicsParamsRef const& p,
+                                 ParticlePhysics const& part,
+                                 std::uint32_t pid,
+                                 std::uint32_t mat,
+                                 double energy,
+                                 double range,
+                                 double step,
+                                 bool apply_cut,
+                                 Engine& rng)
+{
+    phys::GridPoint gp(energy);
+    return calc_eloss(p, part, pid, mat, gp, range, step, apply_cut, rng);
+}
+
 //---------------------------------------------------------------------------//
 // URBAN MULTIPLE SCATTERING
 //---------------------------------------------------------------------------//
@@ -304,12 +320,22 @@ struct MscTrack
     double energy;
     double range;  //!< physics range at the pre-step energy
     double lambda;  //!< transport MFP at the pre-step energy
+    double loge{mth::log(energy)};  //!< of the pre-step energy
 
-    CELER_FUNCTION double calc_msc_mfp(double e) const
+    //! The pre-step energy as a grid point (its log is taken once)
+    CELER_FORCEINLINE_FUNCTION phys::GridPoint pre_step() const
+    {
+        return phys::GridPoint(energy, loge);
+    }
+    CELER_FUNCTION double calc_msc_mfp(phys::GridPoint gp) const
     {
         XsGrid const& g = p.grids[p.msc.xs_grid + 2 * mat + par];
-        double const xsec = phys::calc_grid(g, p.grid_reals, e) / (e * e);
+        double const xsec = phys::calc_grid(g, p.grid_reals, gp) / (gp.energy * gp.energy);
         return 1 / xsec;
+    }
+    CELER_FUNCTION double calc_msc_mfp(double e) const
+    {
+        return this->calc_msc_mfp(phys::GridPoint(e));
     }
     CELER_FUNCTION double calc_inverse_range(double r) const
     {
@@ -324,7 +350,9 @@ struct MscTrack
     {
         if (step <= range * msc_dtrl)
         {
-            double const dedx = phys::calc_grid(p.grids[part.dedx_grid + mat], p.grid_reals, energy);
+            phys::GridPoint gp = this->pre_step();
+            double const dedx
+                = phys::calc_grid(p.grids[part.dedx_grid + mat], p.grid_reals, gp);
             return energy - step * dedx;
         }
         return calc_inverse_range(range - step);

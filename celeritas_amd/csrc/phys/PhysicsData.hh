@@ -54,11 +54,13 @@ struct XsGrid
 {
     double loge_front;  //!< log(E_min / MeV)
     double loge_back;  //!< log(E_max / MeV)
-    double loge_delta;
+    double inv_delta;  //!< points per unit of log(E)
     std::uint32_t size;  //!< number of points (0: no grid)
     std::uint32_t prime_index;  //!< values at i >= prime are scaled by E
     std::uint32_t offset;  //!< into the reals array
-    std::uint32_t pad_;
+    //! Offset of the grid's energies [MeV] in the reals array (grids with
+    //! the same points share them)
+    std::uint32_t energies;
 };
 
 //! One model of a process with its lower energy bound

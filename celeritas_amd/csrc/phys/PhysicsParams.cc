@@ -10,6 +10,7 @@
 #include <type_traits>
 #include <cmath>
 #include <map>
+#include <tuple>
 
 #include "global/ActionInterface.hh"
 #include "PhysicsActions.hh"
@@ -231,7 +232,10 @@ struct PhysicsParams::HostData
 {
     std::vector<ParticlePhysics> particle;
     std::vector<XsGrid> grids;
-    std::vector<double> grid_reals;  //!< XsGrid values and energy_max_xs
+    //! XsGrid values and energies, energy_max_xs
+    std::vector<double> grid_reals;
+    //! (front, delta, size) of the grids whose energies are in grid_reals
+    std::map<std::tuple<double, double, std::uint32_t>, std::uint32_t> energies;
     std::vector<double> reals;  //!< SB and Livermore tables
     std::vector<double> mass;
     std::vector<double> charge;
@@ -325,13 +329,28 @@ struct PhysicsParams::HostData
             XsGrid x{};
             x.loge_front = g.front;
             x.loge_back = g.back;
-            x.loge_delta = g.delta;
+            x.inv_delta = 1 / g.delta;
             x.size = static_cast<std::uint32_t>(g.values.size());
             x.prime_index = g.prime;
             x.offset = static_cast<std::uint32_t>(grid_reals.size());
             grid_reals.insert(grid_reals.end(), g.values.begin(), g.values.end());
+            x.energies = this->add_energies(g.front, g.delta, x.size);
             grids.push_back(x);
         }
+        return first;
+    }
+
+    //! Offset of the energies of a log-uniform grid, shared between grids
+    std::uint32_t add_energies(double front, double delta, std::uint32_t size)
+    {
+        auto const key = std::make_tuple(front, delta, size);
+        auto const iter = energies.find(key);
+        if (iter != energies.end())
+            return iter->second;
+        auto const first = static_cast<std::uint32_t>(grid_reals.size());
+        for (std::uint32_t i = 0; i < size; ++i)
+            grid_reals.push_back(std::exp(front + delta * i));
+        energies.emplace(key, first);
         return first;
     }
 
