@@ -47,6 +47,7 @@ enum VolumeFlags : std::uint8_t
     internal_surfaces = 1,  //!< Crossing a face may keep the track inside
     implicit_vol = 2,  //!< Background: enters any volume via its faces
     simple_safety = 4,  //!< All faces support the normal-distance safety
+    conjunction = 8,  //!< Logic is one sense of every face (vol_senses)
 };
 
 //! Maximum faces per volume: senses fit in one 32-bit mask
@@ -107,6 +108,8 @@ struct GeoParamsRef
     std::uint16_t const* vol_logic_size{nullptr};
     std::int32_t const* logic{nullptr};
     std::uint8_t const* vol_flags{nullptr};
+    //! Inside senses of a conjunction's faces, one bit each
+    std::uint32_t const* vol_senses{nullptr};
     double const* vol_bbox{nullptr};  //!< [lo xyz, hi xyz] per volume
 
     // Connectivity: volumes that have each surface as a face

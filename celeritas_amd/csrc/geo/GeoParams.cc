@@ -306,6 +306,65 @@ GeoInput geo_input_from_orange_json(JsonValue const& doc)
 }
 
 //---------------------------------------------------------------------------//
+namespace
+{
+/*!
+ * Whether a volume's postfix logic is a conjunction that holds each of its
+ * (distinct) faces once, as is or negated, and the senses it asks for.
+ */
+bool conjunction_senses(GeoInput::Volume const& vol, std::uint32_t* senses)
+{
+    struct Term
+    {
+        std::uint32_t faces;
+        std::uint32_t senses;
+    };
+    auto const nf = vol.faces.size();
+    for (std::size_t i = 0; i < nf; ++i)
+    {
+        if (std::count(vol.faces.begin(), vol.faces.end(), vol.faces[i]) != 1)
+            return false;
+    }
+    std::vector<Term> stack;
+    for (auto t : vol.logic)
+    {
+        if (t >= 0)
+        {
+            std::uint32_t const bit = std::uint32_t(1) << t;
+            stack.push_back({bit, bit});
+        }
+        else if (t == logic::lnot && !stack.empty())
+        {
+            // Only a single face's sense can be turned
+            Term& s = stack.back();
+            if (s.faces & (s.faces - 1))
+                return false;
+            s.senses ^= s.faces;
+        }
+        else if (t == logic::land && stack.size() >= 2)
+        {
+            Term const b = stack.back();
+            stack.pop_back();
+            Term& a = stack.back();
+            if (a.faces & b.faces)
+                return false;
+            a = {a.faces | b.faces, a.senses | b.senses};
+        }
+        else
+        {
+            return false;
+        }
+    }
+    std::uint32_t const all = nf >= 32 ? ~std::uint32_t(0)
+                                       : (std::uint32_t(1) << nf) - 1;
+    if (stack.size() != 1 || stack.back().faces != all)
+        return false;
+    *senses = stack.back().senses;
+    return true;
+}
+}  // namespace
+
+//---------------------------------------------------------------------------//
 GeoParams::GeoParams(GeoInput const& inp)
 {
     num_surfaces_ = static_cast<size_type>(inp.surf_types.size());
@@ -354,7 +413,11 @@ GeoParams::GeoParams(GeoInput const& inp)
         std::uint8_t flags = vol.flags;
         if (simple && !(flags & implicit_vol))
             flags |= simple_safety;
+        std::uint32_t senses = 0;
+        if (conjunction_senses(vol, &senses))
+            flags |= conjunction;
         h_flags.push_back(flags);
+        h_senses.push_back(senses);
         if (vol.background)
             background = v;
         labels_.push_back(vol.label);
@@ -466,6 +529,7 @@ GeoParams::GeoParams(GeoInput const& inp)
     std::size_t const o_logic_size = place(h_logic_size);
     std::size_t const o_logic = place(h_logic);
     std::size_t const o_flags = place(h_flags);
+    std::size_t const o_senses = place(h_senses);
     std::size_t const o_bbox = place(h_bbox);
     std::size_t const o_conn_begin = place(h_conn_begin);
     std::size_t const o_conn_size = place(h_conn_size);
@@ -496,6 +560,7 @@ GeoParams::GeoParams(GeoInput const& inp)
     ref_.vol_logic_size = at(o_logic_size, h_logic_size);
     ref_.logic = at(o_logic, h_logic);
     ref_.vol_flags = at(o_flags, h_flags);
+    ref_.vol_senses = at(o_senses, h_senses);
     ref_.vol_bbox = at(o_bbox, h_bbox);
     ref_.conn_begin = at(o_conn_begin, h_conn_begin);
     ref_.conn_size = at(o_conn_size, h_conn_size);

@@ -76,6 +76,7 @@ class GeoParams
     std::vector<std::uint16_t> h_logic_size;
     std::vector<std::int32_t> h_logic;
     std::vector<std::uint8_t> h_flags;
+    std::vector<std::uint32_t> h_senses;
     std::vector<double> h_bbox;
     std::vector<std::uint32_t> h_conn_begin;
     std::vector<std::uint32_t> h_conn_size;

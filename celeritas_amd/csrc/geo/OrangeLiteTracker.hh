@@ -703,6 +703,42 @@ CELER_FORCEINLINE_FUNCTION void move_internal(GeoTrack& g, double const* x)
 }
 
 /*!
+ * Whether a point on a surface, on the given side of it, lies inside a
+ * volume that has the surface as a face.
+ *
+ * A conjunction (every convex cell) is left at its first face with the
+ * other sense, from the last face on: the planes that many cells share come
+ * first, and the point is on one of them. A crossing of the barrel's end
+ * plane tries up to 60 shells whose boxes all hold the point, each with
+ * four faces and a logic program of eight tokens: boundary crossings of the
+ * first 24 steps of 3,000 primaries 147 -> 66 us a step.
+ */
+CELER_FUNCTION bool is_behind(GeoParamsRef const& p,
+                              std::uint32_t vol,
+                              std::uint32_t surf,
+                              bool sense,
+                              double const* x)
+{
+    if (p.vol_flags[vol] & conjunction)
+    {
+        std::uint32_t const begin = p.vol_face_begin[vol];
+        std::uint32_t const senses = p.vol_senses[vol];
+        for (int f = p.vol_num_faces[vol] - 1; f >= 0; --f)
+        {
+            std::uint32_t const s = p.faces[begin + f];
+            bool const side = s == surf ? sense : calc_sense(p, s, x) >= 0;
+            if (side != ((senses >> f) & 1u))
+                return false;
+        }
+        return true;
+    }
+    int on_face;
+    std::uint32_t const mask
+        = calc_sense_mask(p, vol, x, find_face(p, vol, surf), sense, &on_face);
+    return eval_logic(p, vol, mask);
+}
+
+/*!
  * Cross the current surface into the neighboring volume.
  */
 CELER_FUNCTION void cross_boundary(GeoParamsRef const& p, GeoTrack& g)
@@ -727,11 +763,7 @@ CELER_FUNCTION void cross_boundary(GeoParamsRef const& p, GeoTrack& g)
             continue;
         if (cn >= 3 && !in_bbox(p, v, g.pos))
             continue;
-        int const face = find_face(p, v, surf);
-        int on_face;
-        std::uint32_t const mask = calc_sense_mask(
-            p, v, g.pos, face, static_cast<bool>(g.sense), &on_face);
-        if (eval_logic(p, v, mask))
+        if (is_behind(p, v, surf, static_cast<bool>(g.sense), g.pos))
         {
             found = v;
             break;

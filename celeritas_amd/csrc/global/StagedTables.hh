@@ -139,6 +139,7 @@ __device__ __forceinline__ void rebase_geometry(GeoParamsRef* r, char* to)
     r->vol_logic_size = rebase(g.vol_logic_size, from, to);
     r->logic = rebase(g.logic, from, to);
     r->vol_flags = rebase(g.vol_flags, from, to);
+    r->vol_senses = rebase(g.vol_senses, from, to);
     r->vol_bbox = rebase(g.vol_bbox, from, to);
     r->conn_begin = rebase(g.conn_begin, from, to);
     r->conn_size = rebase(g.conn_size, from, to);
