@@ -148,9 +148,7 @@ CELER_FUNCTION void apply_interaction(CoreParamsRef const& params,
     state.particle.energy[slot] = r.energy;
     if (r.action != Interaction::absorbed)
     {
-        geo::GeoTrack g = geo::GeoTrack::load(state.geo, slot);
-        geo::set_dir(params.geo, g, r.dir);
-        g.store(state.geo, slot);
+        geo::set_dir(params.geo, state.geo, slot, r.dir);
     }
     else
     {

@@ -144,7 +144,8 @@ CELER_FORCEINLINE_FUNCTION void along_step_charged_track(CoreParamsRef const& pa
                             && g.pos[2] == orig[2])
                            || !std::isfinite(g.pos[0] + g.pos[1] + g.pos[2])))
         {
-            g.store(state.geo, slot);
+            g.store_moved(state.geo, slot);
+            g.store_turned(state.geo, slot);
             rng.store(state.rng, slot);
             apply_errored(params, state, slot);
             return;
@@ -215,7 +216,8 @@ CELER_FORCEINLINE_FUNCTION void along_step_charged_track(CoreParamsRef const& pa
             geo::move_internal(g, x);
         }
     }
-    g.store(state.geo, slot);
+    g.store_moved(state.geo, slot);
+    g.store_turned(state.geo, slot);
 
     // Time
     double const v = phys::speed(energy, pp.mass[pid]);

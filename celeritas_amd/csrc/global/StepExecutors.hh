@@ -162,7 +162,7 @@ CELER_FUNCTION void along_step_neutral_track(CoreParamsRef const& params,
             geo::move_to_boundary(g);
         else
             geo::move_internal(g, step);
-        g.store(state.geo, slot);
+        g.store_moved(state.geo, slot);
         if (CELER_UNLIKELY(!std::isfinite(g.pos[0] + g.pos[1] + g.pos[2])))
         {
             // Not reachable from a finite FP64 state
@@ -301,7 +301,7 @@ boundary_track(CoreParamsRef const& params, CoreStateRef const& state, size_type
 {
     geo::GeoTrack g = geo::GeoTrack::load(state.geo, slot);
     geo::cross_boundary(params.geo, g);
-    g.store(state.geo, slot);
+    g.store_crossed(state.geo, slot);
     if (g.failed)
     {
         apply_errored(params, state, slot);
