@@ -36,7 +36,7 @@ struct InteractionContext
  * Single-element materials need no draw (PhysicsStepUtils.hh:290-300).
  */
 template<class Engine>
-CELER_FUNCTION std::uint32_t sample_element(PhysicsParamsRef const& p,
+CELER_FORCEINLINE_FUNCTION std::uint32_t sample_element(PhysicsParamsRef const& p,
                                             ProcessRecord const& proc,
                                             std::uint32_t model_index,
                                             std::uint32_t mat,

@@ -27,6 +27,7 @@
 #include "phys/PhysicsImpl.hh"
 #include "track/TrackInitImpl.hh"
 #include "CoreData.hh"
+#include "StepExecutors.hh"
 
 namespace celeritas_amd
 {
@@ -39,7 +40,8 @@ template<bool UseField>
 CELER_FORCEINLINE_FUNCTION void along_step_charged_track(CoreParamsRef const& params,
                                              CoreStateRef const& state,
                                              size_type slot,
-                                             TrackStatus status)
+                                             TrackStatus status,
+                                             bool select = false)
 {
     PhysicsParamsRef const& pp = params.phys;
     PhysicsStateRef const& ps = state.phys;
@@ -50,6 +52,14 @@ CELER_FORCEINLINE_FUNCTION void along_step_charged_track(CoreParamsRef const& pa
     double energy = state.particle.energy[slot];
     std::uint32_t const mat = params.volume_to_material[state.geo.volume[slot]];
     ParticlePhysics const& part = pp.particle[pid];
+    // Everything the track needs is read here, so that the updates at the
+    // end wait for no memory
+    double const time = state.sim.time[slot];
+    double const mfp = ps.interaction_mfp[slot];
+    double const macro_xs = ps.macro_xs[slot];
+    double const deposition = ps.energy_deposition[slot];
+    double const range = ps.dedx_range[slot];
+    std::uint32_t const num_steps = state.sim.num_steps[slot];
     geo::GeoTrack g = geo::GeoTrack::load(state.geo, slot);
     XorwowEngine rng = XorwowEngine::load(state.rng, slot);
 
@@ -64,7 +74,7 @@ CELER_FORCEINLINE_FUNCTION void along_step_charged_track(CoreParamsRef const& pa
     alongstep::MscRange msc_range{ps.msc_range_init[slot], ps.msc_range_factor[slot],
                                   ps.msc_limit_min[slot]};
     alongstep::MscTrack mt{pp, part, mat, pid == pp.electron_id ? 0u : 1u, energy,
-                           ps.dedx_range[slot], 0};
+                           range, 0};
     if (msc_applies)
     {
         mt.lambda = mt.calc_msc_mfp(mt.pre_step());
@@ -205,7 +215,7 @@ CELER_FORCEINLINE_FUNCTION void along_step_charged_track(CoreParamsRef const& pa
         }
         alongstep::MscResult const res = alongstep::msc_scatter(
             mt, pp.materials[mat], pid == pp.positron_id, g.dir, safety, displaced,
-            geom_path, true_path, ps.msc_limit_min[slot], rng);
+            geom_path, true_path, msc_range.limit_min, rng);
         if (res.action != 0)
             geo::set_dir(params.geo, g, res.dir);
         if (res.action == 2)
@@ -222,7 +232,7 @@ CELER_FORCEINLINE_FUNCTION void along_step_charged_track(CoreParamsRef const& pa
     // Time
     double const v = phys::speed(energy, pp.mass[pid]);
     if (v > 0)
-        state.sim.time[slot] += step / v;
+        state.sim.time[slot] = time + step / v;
 
     // Continuous energy loss
     TrackStatus new_status = status;
@@ -233,10 +243,10 @@ CELER_FORCEINLINE_FUNCTION void along_step_charged_track(CoreParamsRef const& pa
             bool const apply_cut = post != params.scalars.boundary_action;
             phys::GridPoint gp = mt.pre_step();
             double const deposited = alongstep::calc_eloss(
-                pp, part, pid, mat, gp, ps.dedx_range[slot], step, apply_cut, rng);
+                pp, part, pid, mat, gp, range, step, apply_cut, rng);
             if (deposited > 0)
             {
-                ps.energy_deposition[slot] += deposited;
+                ps.energy_deposition[slot] = deposition + deposited;
                 energy -= deposited;
 #if CELER_PREC_IS_MIXED
                 if (CELER_UNLIKELY(!(energy >= 0 && energy < HUGE_VAL)))
@@ -262,19 +272,27 @@ CELER_FORCEINLINE_FUNCTION void along_step_charged_track(CoreParamsRef const& pa
             }
         }
     }
-    rng.store(state.rng, slot);
     if (CELER_UNLIKELY(rng.exhausted))
     {
         // A scattering or energy-loss sample was abandoned
+        rng.store(state.rng, slot);
         apply_sampling_failure(params, state, slot);
         return;
     }
 
-    // Interaction MFP and step count
+    // Interaction MFP and step count, and the discrete selection of a track
+    // whose step ends in it (the same draws in the same order as the
+    // action's own launch)
     if (new_status == TrackStatus::alive && post != pp.scalars.discrete_action)
-        ps.interaction_mfp[slot] -= step * ps.macro_xs[slot];
-    state.sim.num_steps[slot] += 1;
+        ps.interaction_mfp[slot] = mfp - step * macro_xs;
+    state.sim.num_steps[slot] = num_steps + 1;
     state.sim.step_length[slot] = step;
+    if (select && post == pp.scalars.discrete_action)
+    {
+        count_selection<true>(state);
+        post = select_discrete(params, state, slot, pid, mat, energy, macro_xs, rng);
+    }
+    rng.store(state.rng, slot);
     state.sim.post_step_action[slot] = post;
 }
 

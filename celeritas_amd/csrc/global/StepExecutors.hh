@@ -21,6 +21,9 @@
 #include <cmath>
 
 #include "corecel/Precision.hh"
+#if CELER_DEVICE_COMPILE
+#    include "corecel/WaveOps.hh"
+#endif
 #include "em/Interactors.hh"
 #include "geo/OrangeLiteTracker.hh"
 #include "phys/PhysicsImpl.hh"
@@ -143,20 +146,143 @@ CELER_FUNCTION void pre_step_track(CoreParamsRef const& params,
 }
 
 //---------------------------------------------------------------------------//
+//! One of four values by selects (a dynamic index would put them in scratch
+//! memory)
+CELER_FORCEINLINE_FUNCTION double
+pick(std::uint32_t i, double a, double b, double c, double d)
+{
+    double const lo = i == 0 ? a : b;
+    double const hi = i == 2 ? c : d;
+    return i < 2 ? lo : hi;
+}
+
+/*!
+ * Discrete selection of a track whose values are at hand: choose the
+ * process by its share of the total cross section, apply the integral-
+ * approach rejection, choose the model by energy and sample the target
+ * element. Returns the post-step action.
+ *
+ * The cross sections of all processes are read together, before the first
+ * comparison: read one by one, each was a memory latency.
+ */
+CELER_FORCEINLINE_FUNCTION std::uint8_t select_discrete(CoreParamsRef const& params,
+                                            CoreStateRef const& state,
+                                            size_type slot,
+                                            std::uint32_t pid,
+                                            std::uint32_t mat,
+                                            double energy,
+                                            double macro_xs,
+                                            XorwowEngine& rng)
+{
+    PhysicsParamsRef const& pp = params.phys;
+    ParticlePhysics const& part = pp.particle[pid];
+    static_assert(max_processes == 4, "one value per process");
+    std::uint32_t const np = part.num_processes;
+    double const* xs = state.phys.per_process_xs + slot;
+    double xs0 = 0, xs1 = 0, xs2 = 0, xs3 = 0;
+    if (np > 0)
+        xs0 = xs[0];
+    if (np > 1)
+        xs1 = xs[state.size];
+    if (np > 2)
+        xs2 = xs[2 * state.size];
+    if (np > 3)
+        xs3 = xs[3 * state.size];
+    state.phys.interaction_mfp[slot] = 0;
+    double accum = -macro_xs * draw_canonical(rng);
+    std::uint32_t pidx = np - 1;
+    bool found = false;
+    for (std::uint32_t i = 0; i + 1 < np && !found; ++i)
+    {
+        accum += pick(i, xs0, xs1, xs2, xs3);
+        found = accum > 0;
+        pidx = found ? i : pidx;
+    }
+    if (CELER_UNLIKELY(!found))
+    {
+        // Falling through to the last process is only correct when it has a
+        // cross section: a draw at the top of [0, 1) with rounding could
+        // otherwise select a process that cannot occur (pair production
+        // below threshold); take the last process that can
+        while (pidx > 0 && !(pick(pidx, xs0, xs1, xs2, xs3) > 0))
+            --pidx;
+    }
+    ProcessRecord const& proc = part.process[pidx];
+    phys::GridPoint gp(energy);
+    if (proc.integral)
+    {
+        double const xs_now = phys::calc_xs(pp, proc, mat, gp);
+        if (draw_canonical(rng) * pick(pidx, xs0, xs1, xs2, xs3) > xs_now)
+            return pp.scalars.integral_rejection_action;
+    }
+    std::uint32_t mi = 0;
+    for (std::uint32_t k = 1; k < proc.num_models; ++k)
+    {
+        if (energy >= proc.models[k].energy_low)
+            mi = k;
+    }
+    state.phys.element[slot]
+        = static_cast<std::uint8_t>(sample_element(pp, proc, mi, mat, gp, rng));
+    return static_cast<std::uint8_t>(proc.models[mi].action);
+}
+
+//! Discrete select of the track in a slot (the action by itself)
+CELER_FUNCTION void discrete_select_track(CoreParamsRef const& params,
+                                          CoreStateRef const& state,
+                                          size_type slot)
+{
+    XorwowEngine rng = XorwowEngine::load(state.rng, slot);
+    std::uint8_t const action
+        = select_discrete(params, state, slot, state.particle.particle_id[slot],
+                          material_of(params, state, slot), state.particle.energy[slot],
+                          state.phys.macro_xs[slot], rng);
+    rng.store(state.rng, slot);
+    state.sim.post_step_action[slot] = action;
+}
+
+//! Count a selection made inside an along-step kernel
+template<bool Charged>
+CELER_FORCEINLINE_FUNCTION void count_selection([[maybe_unused]] CoreStateRef const& state)
+{
+#if CELER_DEVICE_COMPILE
+    if (!state.diag)
+        return;
+    wave::count_active_lanes_spread<diag_spread>(state.diag + diag_discrete * diag_spread);
+    if (Charged)
+    {
+        wave::count_active_lanes_spread<diag_spread>(
+            state.diag + diag_discrete_charged * diag_spread);
+    }
+#endif
+}
+
+//---------------------------------------------------------------------------//
 /*!
  * Neutral along-step: linear propagation to the physics step or the next
- * boundary, time and interaction-MFP updates.
+ * boundary, time and interaction-MFP updates, and with \c select the
+ * discrete selection of a track whose step ends in it (the same draws in
+ * the same order as the action's own launch).
+ *
+ * Everything the track needs is read before the propagation, so that the
+ * updates at the end wait for no memory. CHAIN_FIGURES
  */
 CELER_FUNCTION void along_step_neutral_track(CoreParamsRef const& params,
                                              CoreStateRef const& state,
                                              size_type slot,
-                                             TrackStatus status)
+                                             TrackStatus status,
+                                             bool select = false)
 {
     double step = state.sim.step_length[slot];
     std::uint8_t post = state.sim.post_step_action[slot];
+    std::uint32_t const pid = state.particle.particle_id[slot];
+    double const energy = state.particle.energy[slot];
+    double const macro_xs = state.phys.macro_xs[slot];
+    double const mfp = state.phys.interaction_mfp[slot];
+    double const time = state.sim.time[slot];
+    std::uint32_t const num_steps = state.sim.num_steps[slot];
+    geo::GeoTrack g = geo::GeoTrack::load(state.geo, slot);
     if (step != 0)
     {
-        geo::GeoTrack g = geo::GeoTrack::load(state.geo, slot);
         geo::Propagation prop = geo::find_next_step(params.geo, g, step);
         if (prop.boundary)
             geo::move_to_boundary(g);
@@ -180,90 +306,25 @@ CELER_FUNCTION void along_step_neutral_track(CoreParamsRef const& params,
             post = params.scalars.propagation_limit_action;
         }
         state.sim.step_length[slot] = step;
-        state.sim.post_step_action[slot] = post;
     }
-    if (status == TrackStatus::errored)
-        return;
-    std::uint32_t const pid = state.particle.particle_id[slot];
-    double const v = phys::speed(state.particle.energy[slot], params.phys.mass[pid]);
-    if (v > 0)
-        state.sim.time[slot] += step / v;
-    if (post != params.phys.scalars.discrete_action)
+    if (status != TrackStatus::errored)
     {
-        state.phys.interaction_mfp[slot] -= step * state.phys.macro_xs[slot];
+        double const v = phys::speed(energy, params.phys.mass[pid]);
+        if (v > 0)
+            state.sim.time[slot] = time + step / v;
+        if (post != params.phys.scalars.discrete_action)
+            state.phys.interaction_mfp[slot] = mfp - step * macro_xs;
+        state.sim.num_steps[slot] = num_steps + 1;
     }
-    state.sim.num_steps[slot] += 1;
-}
-
-//---------------------------------------------------------------------------//
-/*!
- * Discrete select: choose the process by its share of the total cross
- * section, apply the integral-approach rejection, choose the model by
- * energy and sample the target element.
- */
-CELER_FUNCTION void discrete_select_track(CoreParamsRef const& params,
-                                          CoreStateRef const& state,
-                                          size_type slot)
-{
-    PhysicsParamsRef const& pp = params.phys;
-    state.phys.interaction_mfp[slot] = 0;
-    std::uint32_t const pid = state.particle.particle_id[slot];
-    ParticlePhysics const& part = pp.particle[pid];
-    std::uint32_t const mat = material_of(params, state, slot);
-    double const energy = state.particle.energy[slot];
-    XorwowEngine rng = XorwowEngine::load(state.rng, slot);
-    double accum = -state.phys.macro_xs[slot] * draw_canonical(rng);
-    std::uint32_t pidx = part.num_processes - 1;
-    bool found = false;
-    for (std::uint32_t i = 0; i + 1 < part.num_processes; ++i)
+    if (select && post == params.phys.scalars.discrete_action)
     {
-        accum += state.phys.per_process_xs[i * state.size + slot];
-        if (accum > 0)
-        {
-            pidx = i;
-            found = true;
-            break;
-        }
+        count_selection<false>(state);
+        XorwowEngine rng = XorwowEngine::load(state.rng, slot);
+        post = select_discrete(params, state, slot, pid,
+                               params.volume_to_material[g.volume], energy, macro_xs, rng);
+        rng.store(state.rng, slot);
     }
-    if (CELER_UNLIKELY(!found))
-    {
-        // Falling through to the last process is only correct when it has a
-        // cross section: a draw at the top of [0, 1) with rounding could
-        // otherwise select a process that cannot occur (pair production
-        // below threshold); take the last process that can
-        while (pidx > 0 && !(state.phys.per_process_xs[pidx * state.size + slot] > 0))
-            --pidx;
-    }
-    ProcessRecord const& proc = part.process[pidx];
-    std::uint8_t action;
-    bool rejected = false;
-    phys::GridPoint gp(energy);
-    if (proc.integral)
-    {
-        double const xs = phys::calc_xs(pp, proc, mat, gp);
-        if (draw_canonical(rng) * state.phys.per_process_xs[pidx * state.size + slot] > xs)
-        {
-            rejected = true;
-        }
-    }
-    if (rejected)
-    {
-        action = pp.scalars.integral_rejection_action;
-    }
-    else
-    {
-        std::uint32_t mi = 0;
-        for (std::uint32_t k = 1; k < proc.num_models; ++k)
-        {
-            if (energy >= proc.models[k].energy_low)
-                mi = k;
-        }
-        state.phys.element[slot]
-            = static_cast<std::uint8_t>(sample_element(pp, proc, mi, mat, gp, rng));
-        action = static_cast<std::uint8_t>(proc.models[mi].action);
-    }
-    rng.store(state.rng, slot);
-    state.sim.post_step_action[slot] = action;
+    state.sim.post_step_action[slot] = post;
 }
 
 //---------------------------------------------------------------------------//

@@ -87,8 +87,8 @@ __global__ void __launch_bounds__(block_size)
         return;
     if (state.diag)
         wave::count_active_lanes_spread<diag_spread>(state.diag + diag_along_neutral * diag_spread);
-    exec::along_step_neutral_track(params, state, slot, status);
-    fused_discrete_select<false>(params, state, slot);
+    exec::along_step_neutral_track(params, state, slot, status,
+                                   params.scalars.fuse_discrete_select);
 }
 
 //---------------------------------------------------------------------------//
