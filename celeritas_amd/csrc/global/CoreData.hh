@@ -128,7 +128,7 @@ struct InitStateRef
 {
     std::uint32_t* vacancies{nullptr};
     std::uint32_t* secondary_counts{nullptr};  //!< size+1
-    std::uint32_t* indices{nullptr};
+    std::uint32_t* indices{nullptr};  //!< scratch: order of initializers, IDs
     std::uint32_t* track_counters{nullptr};  //!< per event
     //! Per event: initializers plus live tracks (0 once the event is done)
     std::int32_t* event_live{nullptr};
@@ -140,7 +140,8 @@ struct InitStateRef
     size_type capacity{0};
     size_type max_events{0};
     //! 1 if event_live and event_edep are maintained (per-event completion
-    //! for the serving loop); plain transport skips their atomics
+    //! for the serving loop, which also reserves track IDs with their sums);
+    //! plain transport skips their atomics
     std::uint32_t event_tally{0};
 };
 

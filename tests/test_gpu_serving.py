@@ -69,6 +69,22 @@ def test_events_overlap(amd, params):
     assert np.sum(r["admit"] <= first_done) >= 2
 
 
+@pytest.mark.parametrize("slots", [1000, 1 << 14])
+def test_tally_of_more_events_than_bins(amd, params, slots):
+    """Events 1,024 apart share a bin of the workgroups' sums (those that
+    come second add to memory directly), and the last chunk of slots is
+    partly filled: no deposit and no track is lost."""
+    server = serving.Server(params, slots)
+    events = wl.served_events(1100, seed=17, nmin=1, nmax=2, emin=100.0, emax=200.0)
+    r = server.run(events, np.zeros(len(events)), max_steps=200_000)
+    assert np.all(r["done"] >= r["admit"])
+    assert r["edep"].sum() == pytest.approx(server.state.get("calo_edep", 100).sum(),
+                                            rel=1e-12)
+    if slots >= 1 << 14:
+        # All fit at once, so such pairs were in flight together
+        assert np.any(r["admit"][1024:] <= r["done"][:76])
+
+
 def test_device_admission_in_order_within_limit(amd, params):
     """The device admits staged events in arrival order while the queued
     initializers stay within the limit, and an event larger than the limit
