@@ -47,7 +47,7 @@ enum VolumeFlags : std::uint8_t
     internal_surfaces = 1,  //!< Crossing a face may keep the track inside
     implicit_vol = 2,  //!< Background: enters any volume via its faces
     simple_safety = 4,  //!< All faces support the normal-distance safety
-    conjunction = 8,  //!< Logic is one sense of every face (vol_senses)
+    conjunction = 8,  //!< Logic is one sense of every face (senses)
 };
 
 //! Maximum faces per volume: senses fit in one 32-bit mask
@@ -83,33 +83,61 @@ static_assert(sizeof(BihNode) == 24, "BihNode layout");
 
 //---------------------------------------------------------------------------//
 /*!
+ * A surface as tracking reads it: its ID, type and first coefficient, which
+ * is the only one of every type but the general plane.
+ *
+ * Each volume lists copies of its faces' surfaces, so a face is one 16-byte
+ * read whose address only depends on the volume, and a loop over faces reads
+ * one ahead (ID, type and coefficient were three reads, each waiting for the
+ * one before; two safety distances and a step took a third of the charged
+ * along-step's 125,000 cycles a wave: full TestEm3 transport 875 -> 840 ms,
+ * 24 steps of 3,000 barrel primaries 13.2 -> 12.4 ms).
+ */
+struct alignas(16) SurfaceRecord
+{
+    double coeff;
+    std::uint32_t id;
+    SurfaceType type;
+    std::uint8_t pad_[3];
+};
+static_assert(sizeof(SurfaceRecord) == 16, "SurfaceRecord layout");
+
+//! What tracking reads of a volume
+struct alignas(16) VolumeRecord
+{
+    std::uint32_t face_begin;  //!< into faces
+    std::uint32_t logic_begin;  //!< into logic
+    std::uint32_t senses;  //!< inside senses of a conjunction's faces
+    std::uint16_t logic_size;
+    std::uint8_t num_faces;
+    std::uint8_t flags;
+};
+static_assert(sizeof(VolumeRecord) == 16, "VolumeRecord layout");
+
+//---------------------------------------------------------------------------//
+/*!
  * Immutable geometry data (device pointers).
  */
 struct GeoParamsRef
 {
     size_type num_surfaces{0};
     size_type num_volumes{0};
-    //! Contiguous region of the surface, face, logic, box and connectivity
-    //! tables (what a tracking kernel can stage in LDS)
+    //! Contiguous region of the tables that a tracking kernel can stage in
+    //! LDS: first those that finding distances reads (track_bytes), then
+    //! those that only a boundary crossing reads
     char const* hot_base{nullptr};
+    std::uint32_t track_bytes{0};
     std::uint32_t hot_bytes{0};
 
-    // Surfaces
-    std::uint8_t const* surf_type{nullptr};
+    // Surfaces; the coefficients are read for general planes only
+    SurfaceRecord const* surfaces{nullptr};
     std::uint32_t const* surf_offset{nullptr};  //!< into surf_data
     double const* surf_data{nullptr};
 
     // Volumes
-    std::uint32_t const* vol_face_begin{nullptr};  //!< into faces
-    std::uint8_t const* vol_num_faces{nullptr};
-    std::uint8_t const* vol_max_isect{nullptr};
-    std::uint32_t const* faces{nullptr};  //!< global surface IDs
-    std::uint32_t const* vol_logic_begin{nullptr};  //!< into logic
-    std::uint16_t const* vol_logic_size{nullptr};
+    VolumeRecord const* volumes{nullptr};
+    SurfaceRecord const* faces{nullptr};  //!< one more at the end
     std::int32_t const* logic{nullptr};
-    std::uint8_t const* vol_flags{nullptr};
-    //! Inside senses of a conjunction's faces, one bit each
-    std::uint32_t const* vol_senses{nullptr};
     double const* vol_bbox{nullptr};  //!< [lo xyz, hi xyz] per volume
 
     // Connectivity: volumes that have each surface as a face

@@ -374,9 +374,13 @@ GeoParams::GeoParams(GeoInput const& inp)
     // Surfaces
     for (size_type s = 0; s < num_surfaces_; ++s)
     {
-        h_surf_type.push_back(inp.surf_types[s]);
+        auto const& data = inp.surf_data[s];
+        h_surfaces.push_back({data.empty() ? 0.0 : data[0],
+                              s,
+                              static_cast<SurfaceType>(inp.surf_types[s]),
+                              {}});
         h_surf_offset.push_back(static_cast<std::uint32_t>(h_surf_data.size()));
-        for (double d : inp.surf_data[s])
+        for (double d : data)
             h_surf_data.push_back(d);
     }
 
@@ -388,22 +392,17 @@ GeoParams::GeoParams(GeoInput const& inp)
         CELER_VALIDATE(vol.faces.size() <= static_cast<std::size_t>(max_faces),
                        << "volume " << v << " has " << vol.faces.size()
                        << " faces (max " << max_faces << ")");
-        h_face_begin.push_back(static_cast<std::uint32_t>(h_faces.size()));
-        h_num_faces.push_back(static_cast<std::uint8_t>(vol.faces.size()));
-        int max_isect = 0;
-        bool simple = true;
+        VolumeRecord record{};
+        record.face_begin = static_cast<std::uint32_t>(h_faces.size());
+        record.num_faces = static_cast<std::uint8_t>(vol.faces.size());
         for (auto s : vol.faces)
         {
             CELER_VALIDATE(s < num_surfaces_, << "bad face in volume " << v);
-            h_faces.push_back(s);
+            h_faces.push_back(h_surfaces[s]);
             conn[s].push_back(v);
-            auto t = static_cast<SurfaceType>(inp.surf_types[s]);
-            max_isect += (t <= SurfaceType::pz || t == SurfaceType::p) ? 1 : 2;
-            simple = simple && (t != SurfaceType::p || true);
         }
-        h_max_isect.push_back(static_cast<std::uint8_t>(max_isect));
-        h_logic_begin.push_back(static_cast<std::uint32_t>(h_logic.size()));
-        h_logic_size.push_back(static_cast<std::uint16_t>(vol.logic.size()));
+        record.logic_begin = static_cast<std::uint32_t>(h_logic.size());
+        record.logic_size = static_cast<std::uint16_t>(vol.logic.size());
         for (auto t : vol.logic)
         {
             CELER_VALIDATE(t < 0 || t < static_cast<std::int32_t>(vol.faces.size()),
@@ -411,13 +410,12 @@ GeoParams::GeoParams(GeoInput const& inp)
             h_logic.push_back(t);
         }
         std::uint8_t flags = vol.flags;
-        if (simple && !(flags & implicit_vol))
+        if (!(flags & implicit_vol))
             flags |= simple_safety;
-        std::uint32_t senses = 0;
-        if (conjunction_senses(vol, &senses))
+        if (conjunction_senses(vol, &record.senses))
             flags |= conjunction;
-        h_flags.push_back(flags);
-        h_senses.push_back(senses);
+        record.flags = flags;
+        h_volumes.push_back(record);
         if (vol.background)
             background = v;
         labels_.push_back(vol.label);
@@ -483,7 +481,7 @@ GeoParams::GeoParams(GeoInput const& inp)
                 boxes[v].lo[k] = h_bbox[6 * v + k];
                 boxes[v].hi[k] = h_bbox[6 * v + 3 + k];
             }
-            if ((h_flags[v] & implicit_vol) || is_empty(boxes[v]))
+            if ((h_volumes[v].flags & implicit_vol) || is_empty(boxes[v]))
                 continue;
             (is_finite(boxes[v]) ? finite : unbounded).push_back(v);
         }
@@ -507,8 +505,8 @@ GeoParams::GeoParams(GeoInput const& inp)
 
     // Upload. The tables that tracking reads per track (surfaces, faces,
     // volume logic and boxes, surface connectivity) share one contiguous
-    // region that a kernel can copy into LDS and rebase into; the point-
-    // location tree stays apart.
+    // region that a kernel can copy into LDS and rebase into, those of
+    // boundary crossings last; the point-location tree stays apart.
     std::vector<char> hot;
     auto place = [&hot](auto const& v) {
         std::size_t const off = (hot.size() + 15) / 16 * 16;
@@ -518,18 +516,16 @@ GeoParams::GeoParams(GeoInput const& inp)
             std::memcpy(hot.data() + off, v.data(), n);
         return off;
     };
-    std::size_t const o_surf_type = place(h_surf_type);
+    // A loop over faces reads the next one ahead
+    h_faces.push_back({0.0, invalid_id, SurfaceType::px, {}});
+    std::size_t const o_faces = place(h_faces);
+    std::size_t const o_volumes = place(h_volumes);
+    std::size_t const o_surfaces = place(h_surfaces);
     std::size_t const o_surf_offset = place(h_surf_offset);
     std::size_t const o_surf_data = place(h_surf_data);
-    std::size_t const o_face_begin = place(h_face_begin);
-    std::size_t const o_num_faces = place(h_num_faces);
-    std::size_t const o_max_isect = place(h_max_isect);
-    std::size_t const o_faces = place(h_faces);
-    std::size_t const o_logic_begin = place(h_logic_begin);
-    std::size_t const o_logic_size = place(h_logic_size);
     std::size_t const o_logic = place(h_logic);
-    std::size_t const o_flags = place(h_flags);
-    std::size_t const o_senses = place(h_senses);
+    hot.resize((hot.size() + 15) / 16 * 16);
+    std::size_t const track_bytes = hot.size();
     std::size_t const o_bbox = place(h_bbox);
     std::size_t const o_conn_begin = place(h_conn_begin);
     std::size_t const o_conn_size = place(h_conn_size);
@@ -549,18 +545,13 @@ GeoParams::GeoParams(GeoInput const& inp)
     ref_.num_volumes = num_volumes_;
     ref_.hot_base = base;
     ref_.hot_bytes = static_cast<std::uint32_t>(hot.size());
-    ref_.surf_type = at(o_surf_type, h_surf_type);
+    ref_.track_bytes = static_cast<std::uint32_t>(track_bytes);
+    ref_.surfaces = at(o_surfaces, h_surfaces);
     ref_.surf_offset = at(o_surf_offset, h_surf_offset);
     ref_.surf_data = at(o_surf_data, h_surf_data);
-    ref_.vol_face_begin = at(o_face_begin, h_face_begin);
-    ref_.vol_num_faces = at(o_num_faces, h_num_faces);
-    ref_.vol_max_isect = at(o_max_isect, h_max_isect);
+    ref_.volumes = at(o_volumes, h_volumes);
     ref_.faces = at(o_faces, h_faces);
-    ref_.vol_logic_begin = at(o_logic_begin, h_logic_begin);
-    ref_.vol_logic_size = at(o_logic_size, h_logic_size);
     ref_.logic = at(o_logic, h_logic);
-    ref_.vol_flags = at(o_flags, h_flags);
-    ref_.vol_senses = at(o_senses, h_senses);
     ref_.vol_bbox = at(o_bbox, h_bbox);
     ref_.conn_begin = at(o_conn_begin, h_conn_begin);
     ref_.conn_size = at(o_conn_size, h_conn_size);

@@ -65,18 +65,12 @@ class GeoParams
     std::uint32_t find_volume(std::string const& label) const;
 
     // Host copies (also exported for the test harness)
-    std::vector<std::uint8_t> h_surf_type;
+    std::vector<SurfaceRecord> h_surfaces;
     std::vector<std::uint32_t> h_surf_offset;
     std::vector<double> h_surf_data;
-    std::vector<std::uint32_t> h_face_begin;
-    std::vector<std::uint8_t> h_num_faces;
-    std::vector<std::uint8_t> h_max_isect;
-    std::vector<std::uint32_t> h_faces;
-    std::vector<std::uint32_t> h_logic_begin;
-    std::vector<std::uint16_t> h_logic_size;
+    std::vector<SurfaceRecord> h_faces;
+    std::vector<VolumeRecord> h_volumes;
     std::vector<std::int32_t> h_logic;
-    std::vector<std::uint8_t> h_flags;
-    std::vector<std::uint32_t> h_senses;
     std::vector<double> h_bbox;
     std::vector<std::uint32_t> h_conn_begin;
     std::vector<std::uint32_t> h_conn_size;

@@ -148,34 +148,37 @@ struct GeoTrack
 //---------------------------------------------------------------------------//
 //! Quadric value whose sign gives the sense
 CELER_FUNCTION double
-eval_surface(GeoParamsRef const& p, std::uint32_t s, double const* x)
+eval_surface(GeoParamsRef const& p, SurfaceRecord const& s, double const* x)
 {
-    double const* d = p.surf_data + p.surf_offset[s];
-    switch (static_cast<SurfaceType>(p.surf_type[s]))
+    double const c = s.coeff;
+    if (s.type == SurfaceType::p)
+    {
+        double const* d = p.surf_data + p.surf_offset[s.id];
+        return d[0] * x[0] + d[1] * x[1] + d[2] * x[2] - d[3];
+    }
+    switch (s.type)
     {
         case SurfaceType::px:
-            return x[0] - d[0];
+            return x[0] - c;
         case SurfaceType::py:
-            return x[1] - d[0];
+            return x[1] - c;
         case SurfaceType::pz:
-            return x[2] - d[0];
+            return x[2] - c;
         case SurfaceType::cxc:
-            return x[1] * x[1] + x[2] * x[2] - d[0];
+            return x[1] * x[1] + x[2] * x[2] - c;
         case SurfaceType::cyc:
-            return x[0] * x[0] + x[2] * x[2] - d[0];
+            return x[0] * x[0] + x[2] * x[2] - c;
         case SurfaceType::czc:
-            return x[0] * x[0] + x[1] * x[1] - d[0];
+            return x[0] * x[0] + x[1] * x[1] - c;
         case SurfaceType::sc:
-            return x[0] * x[0] + x[1] * x[1] + x[2] * x[2] - d[0];
-        case SurfaceType::p:
-            return d[0] * x[0] + d[1] * x[1] + d[2] * x[2] - d[3];
+            return x[0] * x[0] + x[1] * x[1] + x[2] * x[2] - c;
         default:
             return 0;
     }
 }
 
 CELER_FORCEINLINE_FUNCTION int
-calc_sense(GeoParamsRef const& p, std::uint32_t s, double const* x)
+calc_sense(GeoParamsRef const& p, SurfaceRecord const& s, double const* x)
 {
     return real_to_sense(eval_surface(p, s, x));
 }
@@ -225,22 +228,21 @@ CELER_FORCEINLINE_FUNCTION double component(double const* v, int i)
 
 //! Distances to intersection (up to two; no_intersection when absent)
 CELER_FUNCTION void calc_intersections(GeoParamsRef const& p,
-                                       std::uint32_t s,
+                                       SurfaceRecord const& s,
                                        double const* x,
                                        double const* u,
                                        bool on,
                                        double* out)
 {
     out[0] = out[1] = no_intersection;
-    double const* d = p.surf_data + p.surf_offset[s];
-    auto const t = static_cast<SurfaceType>(p.surf_type[s]);
+    SurfaceType const t = s.type;
     if (t <= SurfaceType::pz)
     {
         int const ax = static_cast<int>(t);
         double const n_dir = component(u, ax);
         if (!on && n_dir != 0)
         {
-            double const dist = (d[0] - component(x, ax)) / n_dir;
+            double const dist = (s.coeff - component(x, ax)) / n_dir;
             if (dist > 0)
                 out[0] = dist;
         }
@@ -248,6 +250,7 @@ CELER_FUNCTION void calc_intersections(GeoParamsRef const& p,
     }
     if (t == SurfaceType::p)
     {
+        double const* d = p.surf_data + p.surf_offset[s.id];
         double const n_dir = d[0] * u[0] + d[1] * u[1] + d[2] * u[2];
         if (!on && n_dir != 0)
         {
@@ -261,7 +264,7 @@ CELER_FUNCTION void calc_intersections(GeoParamsRef const& p,
     if (t == SurfaceType::sc)
     {
         double const half_b = u[0] * x[0] + u[1] * x[1] + u[2] * x[2];
-        double const c = x[0] * x[0] + x[1] * x[1] + x[2] * x[2] - d[0];
+        double const c = x[0] * x[0] + x[1] * x[1] + x[2] * x[2] - s.coeff;
         solve_quadratic(1.0, half_b, c, on, out);
         return;
     }
@@ -278,18 +281,17 @@ CELER_FUNCTION void calc_intersections(GeoParamsRef const& p,
     double const xu = component(x, iu);
     double const xv = component(x, iv);
     double const half_b = uu * xu + uv * xv;
-    double const c = xu * xu + xv * xv - d[0];
+    double const c = xu * xu + xv * xv - s.coeff;
     solve_quadratic(a, half_b, c, on, out);
 }
 
 //! Outward unit normal at a point
 CELER_FUNCTION void calc_normal(GeoParamsRef const& p,
-                                std::uint32_t s,
+                                SurfaceRecord const& s,
                                 double const* x,
                                 double* n)
 {
-    double const* d = p.surf_data + p.surf_offset[s];
-    auto const t = static_cast<SurfaceType>(p.surf_type[s]);
+    SurfaceType const t = s.type;
     n[0] = n[1] = n[2] = 0;
     if (t <= SurfaceType::pz)
     {
@@ -301,6 +303,7 @@ CELER_FUNCTION void calc_normal(GeoParamsRef const& p,
     }
     if (t == SurfaceType::p)
     {
+        double const* d = p.surf_data + p.surf_offset[s.id];
         n[0] = d[0];
         n[1] = d[1];
         n[2] = d[2];
@@ -327,10 +330,20 @@ CELER_FUNCTION void calc_normal(GeoParamsRef const& p,
     n[2] *= inv;
 }
 
-//! Nearest distance to the surface along its normal (orange CalcSafety)
+/*!
+ * Nearest distance to the surface along its normal (orange CalcSafety).
+ *
+ * For a plane normal to an axis the intersection along the normal is this
+ * difference divided by one, or by minus one.
+ */
 CELER_FUNCTION double
-calc_safety_distance(GeoParamsRef const& p, std::uint32_t s, double const* x)
+calc_safety_distance(GeoParamsRef const& p, SurfaceRecord const& s, double const* x)
 {
+    if (s.type <= SurfaceType::pz)
+    {
+        double const d = std::fabs(component(x, static_cast<int>(s.type)) - s.coeff);
+        return d >= 0 ? d : HUGE_VAL;
+    }
     double n[3];
     calc_normal(p, s, x, n);
     if (CELER_UNLIKELY(std::isnan(n[0])))
@@ -367,16 +380,20 @@ CELER_FUNCTION std::uint32_t calc_sense_mask(GeoParamsRef const& p,
                                              bool known_sense,
                                              int* on_face)
 {
-    std::uint32_t const begin = p.vol_face_begin[vol];
-    int const nf = p.vol_num_faces[vol];
+    VolumeRecord const record = p.volumes[vol];
+    SurfaceRecord const* faces = p.faces + record.face_begin;
+    int const nf = record.num_faces;
     std::uint32_t mask = 0;
     *on_face = -1;
+    SurfaceRecord next = faces[0];
     for (int f = 0; f < nf; ++f)
     {
+        SurfaceRecord const face = next;
+        next = faces[f + 1];
         bool s;
         if (f != known_face)
         {
-            int const ss = calc_sense(p, p.faces[begin + f], x);
+            int const ss = calc_sense(p, face, x);
             s = ss >= 0;
             if (*on_face < 0 && ss == 0)
                 *on_face = f;
@@ -394,8 +411,9 @@ CELER_FUNCTION std::uint32_t calc_sense_mask(GeoParamsRef const& p,
 CELER_FUNCTION bool
 eval_logic(GeoParamsRef const& p, std::uint32_t vol, std::uint32_t senses)
 {
-    std::int32_t const* lg = p.logic + p.vol_logic_begin[vol];
-    int const n = p.vol_logic_size[vol];
+    VolumeRecord const record = p.volumes[vol];
+    std::int32_t const* lg = p.logic + record.logic_begin;
+    int const n = record.logic_size;
     std::uint64_t stack = 0;
     for (int i = 0; i < n; ++i)
     {
@@ -428,15 +446,15 @@ eval_logic(GeoParamsRef const& p, std::uint32_t vol, std::uint32_t senses)
     return stack & 1u;
 }
 
-//! Index of a global surface among the faces of a volume (or -1)
+//! Index of a surface among the faces of a volume (or -1)
 CELER_FUNCTION int
 find_face(GeoParamsRef const& p, std::uint32_t vol, std::uint32_t surf)
 {
-    std::uint32_t const begin = p.vol_face_begin[vol];
-    int const nf = p.vol_num_faces[vol];
-    for (int f = 0; f < nf; ++f)
+    VolumeRecord const record = p.volumes[vol];
+    SurfaceRecord const* faces = p.faces + record.face_begin;
+    for (int f = 0; f < record.num_faces; ++f)
     {
-        if (p.faces[begin + f] == surf)
+        if (faces[f].id == surf)
             return f;
     }
     return -1;
@@ -590,22 +608,21 @@ CELER_FUNCTION Propagation find_next_step(GeoParamsRef const& p,
         return {0, true};
     }
     std::uint32_t const vol = g.volume;
-    std::uint32_t const begin = p.vol_face_begin[vol];
-    int const nf = p.vol_num_faces[vol];
-    int const on_face = g.is_on_boundary() ? find_face(p, vol, g.surface) : -1;
-    bool const simple = !(p.vol_flags[vol] & (internal_surfaces | implicit_vol));
+    VolumeRecord const record = p.volumes[vol];
+    SurfaceRecord const* faces = p.faces + record.face_begin;
+    int const nf = record.num_faces;
+    bool const simple = !(record.flags & (internal_surfaces | implicit_vol));
 
     // Valid candidate intersections of face f, root k (in [0, max_step])
     auto for_each_isect = [&](auto&& visit) {
+        SurfaceRecord next = faces[0];
         for (int f = 0; f < nf; ++f)
         {
-            std::uint32_t const s = p.faces[begin + f];
-            bool const on = (f == on_face);
-            auto const t = static_cast<SurfaceType>(p.surf_type[s]);
-            if (on && (t <= SurfaceType::pz || t == SurfaceType::p))
-                continue;  // single-intersection surface: cannot reintersect
+            SurfaceRecord const face = next;
+            next = faces[f + 1];
+            bool const on = face.id == g.surface;
             double d2[2];
-            calc_intersections(p, s, g.pos, g.dir, on, d2);
+            calc_intersections(p, face, g.pos, g.dir, on, d2);
             for (int k = 0; k < 2; ++k)
             {
                 double const d = d2[k];
@@ -633,13 +650,13 @@ CELER_FUNCTION Propagation find_next_step(GeoParamsRef const& p,
         });
         if (best_face >= 0)
         {
-            std::uint32_t const s = p.faces[begin + best_face];
+            SurfaceRecord const s = faces[best_face];
             bool cur_sense;
-            if (s == g.surface)
+            if (s.id == g.surface)
                 cur_sense = g.sense;
             else
                 cur_sense = calc_sense(p, s, g.pos) >= 0;
-            isect_surf = s;
+            isect_surf = s.id;
             isect_sense = cur_sense;
             isect_dist = best;
         }
@@ -652,6 +669,7 @@ CELER_FUNCTION Propagation find_next_step(GeoParamsRef const& p,
         // found by a fresh scan each time, so no per-lane intersection list
         // is kept (the usual exit is the first or second candidate).
         int dummy;
+        int const on_face = g.is_on_boundary() ? find_face(p, vol, g.surface) : -1;
         std::uint32_t senses = calc_sense_mask(
             p, vol, g.pos, on_face, static_cast<bool>(g.sense), &dummy);
         double last_d = -1;
@@ -677,7 +695,7 @@ CELER_FUNCTION Propagation find_next_step(GeoParamsRef const& p,
             if (!eval_logic(p, vol, senses))
             {
                 bool const new_sense = (senses >> f) & 1u;
-                isect_surf = p.faces[begin + f];
+                isect_surf = faces[f].id;
                 isect_sense = !new_sense;
                 isect_dist = next_d;
                 break;
@@ -754,15 +772,15 @@ CELER_FUNCTION bool is_behind(GeoParamsRef const& p,
                               bool sense,
                               double const* x)
 {
-    if (p.vol_flags[vol] & conjunction)
+    VolumeRecord const record = p.volumes[vol];
+    if (record.flags & conjunction)
     {
-        std::uint32_t const begin = p.vol_face_begin[vol];
-        std::uint32_t const senses = p.vol_senses[vol];
-        for (int f = p.vol_num_faces[vol] - 1; f >= 0; --f)
+        SurfaceRecord const* faces = p.faces + record.face_begin;
+        for (int f = record.num_faces - 1; f >= 0; --f)
         {
-            std::uint32_t const s = p.faces[begin + f];
-            bool const side = s == surf ? sense : calc_sense(p, s, x) >= 0;
-            if (side != ((senses >> f) & 1u))
+            SurfaceRecord const s = faces[f];
+            bool const side = s.id == surf ? sense : calc_sense(p, s, x) >= 0;
+            if (side != ((record.senses >> f) & 1u))
                 return false;
         }
         return true;
@@ -823,7 +841,7 @@ set_dir(GeoParamsRef const& p, GeoTrack& g, double const* newdir)
     if (g.is_on_boundary())
     {
         double n[3];
-        calc_normal(p, g.surface, g.pos, n);
+        calc_normal(p, p.surfaces[g.surface], g.pos, n);
         double const dn_new = n[0] * newdir[0] + n[1] * newdir[1]
                               + n[2] * newdir[2];
         double const dn_old = n[0] * g.dir[0] + n[1] * g.dir[1]
@@ -851,7 +869,7 @@ CELER_FUNCTION void set_dir(GeoParamsRef const& p,
         double x[3], n[3];
         for (int k = 0; k < 3; ++k)
             x[k] = s.pos[k][i];
-        calc_normal(p, surface, x, n);
+        calc_normal(p, p.surfaces[surface], x, n);
         double const dn_new = n[0] * newdir[0] + n[1] * newdir[1]
                               + n[2] * newdir[2];
         double const dn_old = n[0] * s.dir[0][i] + n[1] * s.dir[1][i]
@@ -869,15 +887,17 @@ CELER_FUNCTION void set_dir(GeoParamsRef const& p,
  */
 CELER_FUNCTION double find_safety(GeoParamsRef const& p, GeoTrack const& g)
 {
-    std::uint32_t const vol = g.volume;
-    if (!(p.vol_flags[vol] & simple_safety))
+    VolumeRecord const record = p.volumes[g.volume];
+    if (!(record.flags & simple_safety))
         return 0;
-    std::uint32_t const begin = p.vol_face_begin[vol];
-    int const nf = p.vol_num_faces[vol];
+    SurfaceRecord const* faces = p.faces + record.face_begin;
     double result = HUGE_VAL;
-    for (int f = 0; f < nf; ++f)
+    SurfaceRecord next = faces[0];
+    for (int f = 0; f < record.num_faces; ++f)
     {
-        double const d = calc_safety_distance(p, p.faces[begin + f], g.pos);
+        SurfaceRecord const face = next;
+        next = faces[f + 1];
+        double const d = calc_safety_distance(p, face, g.pos);
         result = d < result ? d : result;
     }
     return result;

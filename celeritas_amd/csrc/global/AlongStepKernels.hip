@@ -20,8 +20,10 @@ namespace
 {
 constexpr int block_size = 256;
 
+// Three waves per SIMD without a field (168 registers; the LDS of the staged
+// tables allows no more)
 template<bool UseField, Staging S>
-__global__ void __launch_bounds__(block_size)
+__global__ void __launch_bounds__(block_size, UseField ? 1 : 3)
     along_step_charged_kernel(CoreParamsRef const params_in,
                               CoreStateRef const state,
                               std::uint8_t const action,

@@ -13,7 +13,7 @@
 //! dynamic LDS copies the regions it reads once per workgroup and continues
 //! with a params view whose table pointers are rebased into LDS, so the
 //! chains of dependent table reads of a track (particle -> process -> grid
-//! header -> values; volume -> faces -> surfaces -> coefficients) are served
+//! header -> values; volume -> faces) are served
 //! from LDS instead of L2. The data are the same bytes, so results are
 //! bit-identical to the unstaged path.
 //---------------------------------------------------------------------------//
@@ -45,14 +45,22 @@ inline unsigned int staged_table_bytes(CoreParamsRef const& p)
     return (n > 0 && n <= max_staged_table_bytes) ? n : 0;
 }
 
-//! Dynamic LDS bytes of a launch staging the geometry tables
+//! Dynamic LDS bytes of a launch staging the tables that finding distances
+//! reads
 inline unsigned int staged_geo_bytes(CoreParamsRef const& p)
+{
+    unsigned int const n = p.geo.track_bytes;
+    return (n > 0 && n <= max_staged_table_bytes) ? n : 0;
+}
+
+//! Dynamic LDS bytes of a launch staging all geometry tables
+inline unsigned int staged_crossing_bytes(CoreParamsRef const& p)
 {
     unsigned int const n = p.geo.hot_bytes;
     return (n > 0 && n <= max_staged_table_bytes) ? n : 0;
 }
 
-//! Dynamic LDS bytes of a launch staging both (physics first)
+//! Dynamic LDS bytes of a launch staging physics and distances (physics first)
 inline unsigned int staged_both_bytes(CoreParamsRef const& p)
 {
     unsigned int const a = staged_table_bytes(p);
@@ -65,8 +73,9 @@ enum class Staging
 {
     none,
     physics,
-    geometry,
-    both,
+    geometry,  //!< what finding distances reads
+    crossing,  //!< all of the geometry
+    both,  //!< physics and geometry
 };
 
 /*!
@@ -142,23 +151,24 @@ __device__ __forceinline__ void rebase_physics(PhysicsParamsRef* r, char* to)
     r->model_class = rebase(pp.model_class, from, to);
 }
 
-//! Geometry table pointers rebased into LDS
+//! Pointers of the tables that finding distances reads
 __device__ __forceinline__ void rebase_geometry(GeoParamsRef* r, char* to)
 {
     GeoParamsRef const g = *r;
     char const* from = g.hot_base;
-    r->surf_type = rebase(g.surf_type, from, to);
+    r->surfaces = rebase(g.surfaces, from, to);
     r->surf_offset = rebase(g.surf_offset, from, to);
     r->surf_data = rebase(g.surf_data, from, to);
-    r->vol_face_begin = rebase(g.vol_face_begin, from, to);
-    r->vol_num_faces = rebase(g.vol_num_faces, from, to);
-    r->vol_max_isect = rebase(g.vol_max_isect, from, to);
+    r->volumes = rebase(g.volumes, from, to);
     r->faces = rebase(g.faces, from, to);
-    r->vol_logic_begin = rebase(g.vol_logic_begin, from, to);
-    r->vol_logic_size = rebase(g.vol_logic_size, from, to);
     r->logic = rebase(g.logic, from, to);
-    r->vol_flags = rebase(g.vol_flags, from, to);
-    r->vol_senses = rebase(g.vol_senses, from, to);
+}
+
+//! Pointers of the tables that only boundary crossings read
+__device__ __forceinline__ void rebase_crossing(GeoParamsRef* r, char* to)
+{
+    GeoParamsRef const g = *r;
+    char const* from = g.hot_base;
     r->vol_bbox = rebase(g.vol_bbox, from, to);
     r->conn_begin = rebase(g.conn_begin, from, to);
     r->conn_size = rebase(g.conn_size, from, to);
@@ -174,7 +184,7 @@ __device__ __forceinline__ void rebase_geometry(GeoParamsRef* r, char* to)
  * Every thread of the workgroup must call this before any of them returns
  * (it contains a workgroup barrier). The launcher gives the kernel the
  * LDS its staging needs (staged_table_bytes, staged_geo_bytes,
- * staged_both_bytes) and instantiates it with that staging only when the
+ * staged_crossing_bytes, staged_both_bytes) and instantiates it with that staging only when the
  * regions fit: the table pointers then derive from the LDS array alone,
  * so the compiler reads them with LDS instructions and 32-bit addresses.
  */
@@ -198,8 +208,14 @@ __device__ __forceinline__ CoreParamsRef stage(CoreParamsRef const& params, void
         }
         if constexpr (S == Staging::geometry || S == Staging::both)
         {
-            detail::copy_region(params.geo.hot_base, params.geo.hot_bytes, to + offset);
+            detail::copy_region(params.geo.hot_base, params.geo.track_bytes, to + offset);
             detail::rebase_geometry(&r.geo, to + offset);
+        }
+        if constexpr (S == Staging::crossing)
+        {
+            detail::copy_region(params.geo.hot_base, params.geo.hot_bytes, to);
+            detail::rebase_geometry(&r.geo, to);
+            detail::rebase_crossing(&r.geo, to);
         }
         __syncthreads();
         return r;

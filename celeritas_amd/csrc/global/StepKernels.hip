@@ -68,8 +68,10 @@ __global__ void __launch_bounds__(block_size)
 //---------------------------------------------------------------------------//
 // ALONG-STEP (NEUTRAL)
 //---------------------------------------------------------------------------//
+// Five waves per SIMD; the few registers that takes are in scratch memory
+// where the table pointers are not in LDS, so there it is four
 template<Staging S>
-__global__ void __launch_bounds__(block_size)
+__global__ void __launch_bounds__(block_size, S == Staging::none ? 4 : 5)
     along_step_neutral_kernel(CoreParamsRef const params_in,
                               CoreStateRef const state,
                               std::uint8_t const action,
@@ -429,9 +431,9 @@ hipError_t launch_boundary(CoreParamsRef const& p,
                            ThreadSlots const& ts,
                            hipStream_t st)
 {
-    unsigned int const lds = staged_geo_bytes(p);
+    unsigned int const lds = staged_crossing_bytes(p);
     launch_kernel("boundary",
-                  lds ? boundary_kernel<Staging::geometry> : boundary_kernel<Staging::none>,
+                  lds ? boundary_kernel<Staging::crossing> : boundary_kernel<Staging::none>,
                   grid_of(s), s.block_size, lds, st, p, s, ts);
     return hipGetLastError();
 }
