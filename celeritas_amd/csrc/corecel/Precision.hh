@@ -24,6 +24,7 @@
 #include <cmath>
 #include <cstdint>
 
+#include "Elementary.hh"
 #include "Macros.hh"
 #include "random/XorwowEngine.hh"
 
@@ -120,6 +121,11 @@ CELER_FORCEINLINE_FUNCTION double cos(double x)
 {
     return static_cast<double>(::cosf(static_cast<float>(x)));
 }
+CELER_FORCEINLINE_FUNCTION void sincos(double x, double* s, double* c)
+{
+    *s = mth::sin(x);
+    *c = mth::cos(x);
+}
 CELER_FORCEINLINE_FUNCTION double cbrt(double x)
 {
     return static_cast<double>(::cbrtf(static_cast<float>(x)));
@@ -145,15 +151,16 @@ CELER_FORCEINLINE_FUNCTION double tanh(double x)
     return static_cast<double>(::tanhf(static_cast<float>(x)));
 }
 #else
+using elem::cos;
+using elem::log;
+using elem::sin;
+using elem::sincos;
 using std::atan;
 using std::cbrt;
-using std::cos;
 using std::exp;
 using std::expm1;
-using std::log;
 using std::log1p;
 using std::pow;
-using std::sin;
 using std::sqrt;
 using std::tan;
 using std::tanh;

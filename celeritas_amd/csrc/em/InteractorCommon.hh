@@ -78,10 +78,9 @@ from_spherical(double costheta, double phi, double* out)
     double const sintheta = sin_of_cos(costheta);
     double s, c;
 #if CELER_DEVICE_COMPILE
-    sincos(phi, &s, &c);
+    elem::sincos(phi, &s, &c);
 #else
-    s = mth::sin(phi);
-    c = mth::cos(phi);
+    mth::sincos(phi, &s, &c);
 #endif
     out[0] = sintheta * c;
     out[1] = sintheta * s;

@@ -52,12 +52,9 @@ CELER_FORCEINLINE_FUNCTION void along_step_charged_track(CoreParamsRef const& pa
     double energy = state.particle.energy[slot];
     std::uint32_t const mat = params.volume_to_material[state.geo.volume[slot]];
     ParticlePhysics const& part = pp.particle[pid];
-    // Everything the track needs is read here, so that the updates at the
-    // end wait for no memory
-    double const time = state.sim.time[slot];
+    // Read here, so that the updates at the end wait for no memory
     double const mfp = ps.interaction_mfp[slot];
     double const macro_xs = ps.macro_xs[slot];
-    double const deposition = ps.energy_deposition[slot];
     double const range = ps.dedx_range[slot];
     std::uint32_t const num_steps = state.sim.num_steps[slot];
     geo::GeoTrack g = geo::GeoTrack::load(state.geo, slot);
@@ -229,7 +226,9 @@ CELER_FORCEINLINE_FUNCTION void along_step_charged_track(CoreParamsRef const& pa
     g.store_moved(state.geo, slot);
     g.store_turned(state.geo, slot);
 
-    // Time
+    // Time, and read ahead what follows the energy loss
+    double const deposition = ps.energy_deposition[slot];
+    double const time = state.sim.time[slot];
     double const v = phys::speed(energy, pp.mass[pid]);
     if (v > 0)
         state.sim.time[slot] = time + step / v;

@@ -148,7 +148,7 @@ __global__ void __launch_bounds__(block_size)
  * following one another.
  */
 template<bool Staged>
-__global__ void __launch_bounds__(block_size)
+__global__ void __launch_bounds__(block_size, 3)
     interactions_kernel(CoreParamsRef const params_in,
                         CoreStateRef const state,
                         ThreadSlots const ts)

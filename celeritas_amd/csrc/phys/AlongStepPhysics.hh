@@ -49,9 +49,11 @@ struct Normal
         }
         double const theta = (2 * phys::pi) * draw_canonical(rng);
         double const r = mth::sqrt(-2 * mth::log(draw_canonical(rng)));
-        spare = r * mth::cos(theta);
+        double s, c;
+        mth::sincos(theta, &s, &c);
+        spare = r * c;
         has_spare = true;
-        return std::fma(r * mth::sin(theta), stddev, mean);
+        return std::fma(r * s, stddev, mean);
     }
 };
 
@@ -746,7 +748,9 @@ CELER_FUNCTION MscResult msc_scatter(MscTrack const& t,
             double const cbeta1 = 0.9988703417569197;
             double const psi = -mth::log(1 - draw_canonical(rng) * cbeta1) / cbeta;
             double const dphi = draw_canonical(rng) < 0.5 ? phi + psi : phi - psi;
-            double const local[3] = {mth::cos(dphi), mth::sin(dphi), 0};
+            double local[3];
+            mth::sincos(dphi, &local[1], &local[0]);
+            local[2] = 0;
             rotate(local, inc_dir, result.displacement);
             for (int i = 0; i < 3; ++i)
                 result.displacement[i] *= length;
