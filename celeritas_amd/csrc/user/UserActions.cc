@@ -6,6 +6,9 @@
 #include "UserActions.hh"
 
 #include <algorithm>
+#include <cstring>
+#include <functional>
+#include <type_traits>
 
 #include "global/CoreParams.hh"
 #include "global/CoreState.hh"
@@ -158,12 +161,26 @@ std::vector<std::uint64_t> StepDiagnostic::calc_steps() const
 //---------------------------------------------------------------------------//
 // STEP COLLECTOR
 //---------------------------------------------------------------------------//
+namespace
+{
+//! Words of hits that read() takes through page-locked memory at once (1 MiB:
+//! above it a copy for each column costs less than its bytes)
+constexpr std::uint64_t packed_capacity = (1u << 20) / sizeof(std::uint32_t);
+constexpr std::size_t packed_header = sizeof(StepHitCounters) / sizeof(std::uint32_t);
+
+struct HostFree
+{
+    void operator()(std::uint32_t* p) const { (void)hipHostFree(p); }
+};
+}  // namespace
+
 struct StepCollector::StreamData
 {
     size_type size{0};
     DeviceVector<std::uint32_t> u32;  //!< all 32-bit columns
     DeviceVector<double> f64;  //!< all real columns
     DeviceVector<StepHitCounters> counters;
+    std::unique_ptr<std::uint32_t, HostFree> packed;
     StepCollectorRef ref;
 };
 
@@ -270,6 +287,11 @@ void StepCollector::begin_run(CoreParams const&, CoreState& state)
     u.assign(sd->u32.data());
     if (f.total)
         f.assign(sd->f64.data());
+    std::uint32_t* packed = nullptr;
+    CELER_HIP_CALL(hipHostMalloc(reinterpret_cast<void**>(&packed),
+                                 (packed_header + packed_capacity) * sizeof(std::uint32_t),
+                                 hipHostMallocDefault));
+    sd->packed.reset(packed);
     sd->counters.resize(1);
     r.counters = sd->counters.data();
     CELER_HIP_CALL(launch_step_hits_clear(r.counters, state.stream()));
@@ -291,40 +313,67 @@ DetectorStepOutput StepCollector::read(std::uint32_t stream_id)
     if (iter == streams_.end())
         return out;
     StepCollectorRef const& r = iter->second->ref;
-    CELER_HIP_CALL(hipDeviceSynchronize());
-    StepHitCounters c{};
-    CELER_HIP_CALL(hipMemcpy(&c, r.counters, sizeof(c), hipMemcpyDeviceToHost));
-    std::size_t const n = c.num_hits;
-    auto copy = [n](auto* dst, auto const* src, std::size_t width) {
+    // Columns in reading order
+    StepHitColumns cols;
+    std::vector<std::function<void(std::size_t, std::uint32_t const*)>> fill;
+    auto column = [&](auto* dst, auto const* src, std::uint32_t width) {
         if (!src)
             return;
-        dst->resize(n * width);
-        if (n)
-            CELER_HIP_CALL(hipMemcpy(dst->data(), src, n * width * sizeof((*dst)[0]),
-                                     hipMemcpyDeviceToHost));
+        using T = std::remove_const_t<std::remove_reference_t<decltype(*src)>>;
+        std::uint32_t const words = width * sizeof(T) / sizeof(std::uint32_t);
+        cols.columns[cols.num_columns++]
+            = {reinterpret_cast<std::uint32_t const*>(src), words};
+        // From packed host memory, or without it from the device
+        fill.push_back([dst, src, width](std::size_t n, std::uint32_t const* packed) {
+            dst->resize(n * width);
+            if (n && packed)
+                std::memcpy(dst->data(), packed, n * width * sizeof(T));
+            else if (n)
+                CELER_HIP_CALL(hipMemcpy(dst->data(), src, n * width * sizeof(T),
+                                         hipMemcpyDeviceToHost));
+        });
     };
-    copy(&out.detector, r.hits.detector, 1);
-    copy(&out.track_id, r.hits.track_id, 1);
+    column(&out.detector, r.hits.detector, 1);
+    column(&out.track_id, r.hits.track_id, 1);
     for (int p = 0; p < 2; ++p)
     {
         StepPointHits const& h = r.hits.points[p];
-        copy(&out.points[p].time, h.time, 1);
-        copy(&out.points[p].pos, h.pos, 3);
-        copy(&out.points[p].dir, h.dir, 3);
-        copy(&out.points[p].volume_id, h.volume_id, 1);
-        copy(&out.points[p].energy, h.energy, 1);
+        column(&out.points[p].time, h.time, 1);
+        column(&out.points[p].pos, h.pos, 3);
+        column(&out.points[p].dir, h.dir, 3);
+        column(&out.points[p].volume_id, h.volume_id, 1);
+        column(&out.points[p].energy, h.energy, 1);
     }
-    copy(&out.event_id, r.hits.event_id, 1);
-    copy(&out.parent_id, r.hits.parent_id, 1);
-    copy(&out.track_step_count, r.hits.track_step_count, 1);
-    copy(&out.action_id, r.hits.action_id, 1);
-    copy(&out.step_length, r.hits.step_length, 1);
-    copy(&out.particle, r.hits.particle, 1);
-    copy(&out.energy_deposition, r.hits.energy_deposition, 1);
+    column(&out.event_id, r.hits.event_id, 1);
+    column(&out.parent_id, r.hits.parent_id, 1);
+    column(&out.track_step_count, r.hits.track_step_count, 1);
+    column(&out.action_id, r.hits.action_id, 1);
+    column(&out.step_length, r.hits.step_length, 1);
+    column(&out.particle, r.hits.particle, 1);
+    column(&out.energy_deposition, r.hits.energy_deposition, 1);
+
+    CELER_HIP_CALL(hipDeviceSynchronize());
+    std::uint32_t const* packed = iter->second->packed.get();
+    CELER_HIP_CALL(launch_step_hits_pack(cols, r.counters, packed_capacity,
+                                         iter->second->packed.get(), nullptr));
+    CELER_HIP_CALL(hipDeviceSynchronize());
+    StepHitCounters c{};
+    std::memcpy(&c, packed, sizeof(c));
+    packed += packed_header;
+    bool const fits = packed_words(cols, c.num_hits) <= packed_capacity;
+    for (std::uint32_t i = 0; i < cols.num_columns; ++i)
+    {
+        fill[i](c.num_hits, fits ? packed : nullptr);
+        if (fits)
+            packed += packed_words(cols.columns[i], c.num_hits);
+    }
     out.overflow_steps = c.overflow;
     out.dropped_hits = c.dropped;
-    CELER_HIP_CALL(launch_step_hits_clear(r.counters, nullptr));
-    CELER_HIP_CALL(hipDeviceSynchronize());
+    if (!fits)
+    {
+        CELER_HIP_CALL(launch_step_hits_clear(r.counters, nullptr));
+        CELER_HIP_CALL(hipDeviceSynchronize());
+    }
     return out;
 }
 

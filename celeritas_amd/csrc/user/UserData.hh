@@ -115,6 +115,36 @@ struct StepHitCounters
     std::uint32_t dropped;  //!< hits lost to overflow
 };
 
+//! Selected columns of the hit buffer, as 32-bit words, in reading order
+struct StepHitColumns
+{
+    static constexpr unsigned int max_columns = 20;
+    struct Column
+    {
+        std::uint32_t const* data;
+        std::uint32_t words;  //!< per hit
+    };
+    Column columns[max_columns];
+    std::uint32_t num_columns{0};
+};
+
+//! Words of a packed column (whole 8-byte words, so that reals are aligned)
+CELER_FORCEINLINE_FUNCTION std::uint64_t
+packed_words(StepHitColumns::Column const& c, std::uint32_t num_hits)
+{
+    return (std::uint64_t(c.words) * num_hits + 1) / 2 * 2;
+}
+
+//! Words of all packed columns
+CELER_FORCEINLINE_FUNCTION std::uint64_t
+packed_words(StepHitColumns const& cols, std::uint32_t num_hits)
+{
+    std::uint64_t total = 0;
+    for (std::uint32_t i = 0; i < cols.num_columns; ++i)
+        total += packed_words(cols.columns[i], num_hits);
+    return total;
+}
+
 /*!
  * Shared and per-stream data of the collector (StepParamsData and
  * StepStateData, StepData.hh:124-340).

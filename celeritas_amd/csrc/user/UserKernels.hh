@@ -30,4 +30,10 @@ hipError_t launch_step_gather_post(CoreParamsRef const&,
                                    hipStream_t);
 //! Empty the hit buffer and its overflow counters
 hipError_t launch_step_hits_clear(StepHitCounters*, hipStream_t);
+//! Pack the hits to host memory and, if they fit, empty the buffer
+hipError_t launch_step_hits_pack(StepHitColumns const&,
+                                 StepHitCounters*,
+                                 std::uint64_t capacity,
+                                 std::uint32_t* out,
+                                 hipStream_t);
 }  // namespace celeritas_amd

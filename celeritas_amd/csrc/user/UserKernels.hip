@@ -291,6 +291,50 @@ __global__ void step_hits_clear_kernel(StepHitCounters* c)
     c->dropped = 0;
 }
 
+/*!
+ * Write the counters (four words) and, if they fit in \c capacity words, the
+ * selected columns one after the other to memory of the host.
+ *
+ * Bound by round trips: a copy for each column, each waiting for the one
+ * before, took 25 us whatever its size (nine columns and the counters read
+ * after each of 20 steps: steps and hits together 8.7 -> 6.1 ms).
+ */
+__global__ void __launch_bounds__(block_size)
+    step_hits_pack_kernel(StepHitColumns const cols,
+                          StepHitCounters const* counters,
+                          std::uint64_t capacity,
+                          std::uint32_t* out)
+{
+    std::uint32_t const n = counters->num_hits;
+    std::uint32_t const tid = blockIdx.x * block_size + threadIdx.x;
+    if (tid == 0)
+        *reinterpret_cast<StepHitCounters*>(out) = *counters;
+    if (packed_words(cols, n) > capacity)
+        return;
+    std::uint32_t* dst = out + sizeof(StepHitCounters) / sizeof(std::uint32_t);
+    for (std::uint32_t c = 0; c < cols.num_columns; ++c)
+    {
+        std::uint64_t const words = std::uint64_t(cols.columns[c].words) * n;
+        std::uint32_t const* src = cols.columns[c].data;
+        for (std::uint64_t i = tid; i < words; i += gridDim.x * block_size)
+            dst[i] = src[i];
+        dst += packed_words(cols.columns[c], n);
+    }
+}
+
+//! Empty the hit buffer after step_hits_pack_kernel if its columns fitted
+__global__ void step_hits_clear_packed_kernel(StepHitColumns const cols,
+                                              StepHitCounters* c,
+                                              std::uint64_t capacity)
+{
+    if (packed_words(cols, c->num_hits) > capacity)
+        return;
+    c->num_hits = 0;
+    c->step_hits = 0;
+    c->overflow = 0;
+    c->dropped = 0;
+}
+
 unsigned int blocks_of(size_type n)
 {
     return (n + block_size - 1) / block_size;
@@ -345,6 +389,17 @@ hipError_t launch_step_gather_post(CoreParamsRef const& params,
     step_gather_count_kernel<<<nb, block_size, 0, stream>>>(state, coll);
     step_gather_scan_kernel<<<1, 1024, 0, stream>>>(coll, nb);
     step_gather_scatter_kernel<<<nb, block_size, 0, stream>>>(params, state, coll);
+    return hipGetLastError();
+}
+
+hipError_t launch_step_hits_pack(StepHitColumns const& cols,
+                                 StepHitCounters* counters,
+                                 std::uint64_t capacity,
+                                 std::uint32_t* out,
+                                 hipStream_t stream)
+{
+    step_hits_pack_kernel<<<64, block_size, 0, stream>>>(cols, counters, capacity, out);
+    step_hits_clear_packed_kernel<<<1, 1, 0, stream>>>(cols, counters, capacity);
     return hipGetLastError();
 }
 

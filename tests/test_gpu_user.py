@@ -173,3 +173,37 @@ def test_hit_buffer_overflow_and_graph_replay(amd, testem3):
     assert small["overflow_steps"] > 0
     assert n + small["dropped_hits"] == len(eager["detector"])
     assert n <= 64
+
+
+@pytest.mark.parametrize("primaries, steps", [(8, 12), (64, 24)])
+def test_hits_read_at_once_or_by_column(amd, testem3, primaries, steps):
+    """Hits read each step (a few, packed through host memory in one go) and
+    all together at the end (with 64 primaries over 1 MiB: a copy for each
+    column) are the same; an odd count leaves reals aligned."""
+    dets = _gap_detectors(testem3)
+    prim = wl.testem3_primaries(primaries, emin=1e3, emax=1e4, seed=6)
+
+    def run(each):
+        params = amd.CoreParams(testem3)
+        coll = user.StepCollector(params, user.StepSelection.all(), volume_to_detector=dets,
+                                  hit_capacity=1 << 18)
+        stepper = amd.Stepper(params, 1 << 15)
+        stepper.reseed(3)
+        out = []
+        for step in range(steps):
+            stepper(prim) if step == 0 else stepper()
+            if each or step == steps - 1:
+                out.append(coll.read())
+        assert len(coll.read()["detector"]) == 0
+        assert all(h["overflow_steps"] == 0 for h in out)
+        return {c: np.concatenate([h[c] for h in out]) for c in INT_COLUMNS + REAL_COLUMNS}
+
+    each, last = run(True), run(False)
+    n = len(each["detector"])
+    if primaries == 64:
+        assert n * 180 > 1 << 20
+    assert n > 0
+    for c in each:
+        if c in ("track_id", "parent_id"):  # from an atomic counter
+            continue
+        np.testing.assert_array_equal(each[c], last[c], err_msg=c)
