@@ -32,7 +32,7 @@ CELER_FORCEINLINE_FUNCTION int surface_data_size(SurfaceType t)
     return t == SurfaceType::p ? 4 : 1;
 }
 
-//! Logic tokens (postfix); values below lbegin are face indices
+//! Logic tokens (postfix); the others are face indices
 namespace logic
 {
 inline constexpr std::int32_t ltrue = -3;
@@ -83,8 +83,8 @@ static_assert(sizeof(BihNode) == 24, "BihNode layout");
 
 //---------------------------------------------------------------------------//
 /*!
- * A surface as tracking reads it: its ID, type and first coefficient, which
- * is the only one of every type but the general plane.
+ * A surface as tracking reads it: its ID, type and coefficient. Every type
+ * has one but the general plane, whose record holds its place in planes.
  *
  * Each volume lists copies of its faces' surfaces, so a face is one 16-byte
  * read whose address only depends on the volume, and a loop over faces reads
@@ -129,15 +129,14 @@ struct GeoParamsRef
     std::uint32_t track_bytes{0};
     std::uint32_t hot_bytes{0};
 
-    // Surfaces; the coefficients are read for general planes only
+    // Surfaces
     SurfaceRecord const* surfaces{nullptr};
-    std::uint32_t const* surf_offset{nullptr};  //!< into surf_data
-    double const* surf_data{nullptr};
+    double const* planes{nullptr};  //!< {nx, ny, nz, d} per general plane
 
     // Volumes
     VolumeRecord const* volumes{nullptr};
     SurfaceRecord const* faces{nullptr};  //!< one more at the end
-    std::int32_t const* logic{nullptr};
+    std::int8_t const* logic{nullptr};
     double const* vol_bbox{nullptr};  //!< [lo xyz, hi xyz] per volume
 
     // Connectivity: volumes that have each surface as a face

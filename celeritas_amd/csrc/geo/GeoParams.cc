@@ -375,13 +375,14 @@ GeoParams::GeoParams(GeoInput const& inp)
     for (size_type s = 0; s < num_surfaces_; ++s)
     {
         auto const& data = inp.surf_data[s];
-        h_surfaces.push_back({data.empty() ? 0.0 : data[0],
-                              s,
-                              static_cast<SurfaceType>(inp.surf_types[s]),
-                              {}});
-        h_surf_offset.push_back(static_cast<std::uint32_t>(h_surf_data.size()));
-        for (double d : data)
-            h_surf_data.push_back(d);
+        auto const type = static_cast<SurfaceType>(inp.surf_types[s]);
+        double coeff = data.empty() ? 0.0 : data[0];
+        if (type == SurfaceType::p)
+        {
+            coeff = static_cast<double>(h_planes.size() / 4);
+            h_planes.insert(h_planes.end(), data.begin(), data.end());
+        }
+        h_surfaces.push_back({coeff, s, type, {}});
     }
 
     // Volumes
@@ -407,7 +408,7 @@ GeoParams::GeoParams(GeoInput const& inp)
         {
             CELER_VALIDATE(t < 0 || t < static_cast<std::int32_t>(vol.faces.size()),
                            << "bad logic token in volume " << v);
-            h_logic.push_back(t);
+            h_logic.push_back(static_cast<std::int8_t>(t));
         }
         std::uint8_t flags = vol.flags;
         if (!(flags & implicit_vol))
@@ -521,8 +522,7 @@ GeoParams::GeoParams(GeoInput const& inp)
     std::size_t const o_faces = place(h_faces);
     std::size_t const o_volumes = place(h_volumes);
     std::size_t const o_surfaces = place(h_surfaces);
-    std::size_t const o_surf_offset = place(h_surf_offset);
-    std::size_t const o_surf_data = place(h_surf_data);
+    std::size_t const o_planes = place(h_planes);
     std::size_t const o_logic = place(h_logic);
     hot.resize((hot.size() + 15) / 16 * 16);
     std::size_t const track_bytes = hot.size();
@@ -547,8 +547,7 @@ GeoParams::GeoParams(GeoInput const& inp)
     ref_.hot_bytes = static_cast<std::uint32_t>(hot.size());
     ref_.track_bytes = static_cast<std::uint32_t>(track_bytes);
     ref_.surfaces = at(o_surfaces, h_surfaces);
-    ref_.surf_offset = at(o_surf_offset, h_surf_offset);
-    ref_.surf_data = at(o_surf_data, h_surf_data);
+    ref_.planes = at(o_planes, h_planes);
     ref_.volumes = at(o_volumes, h_volumes);
     ref_.faces = at(o_faces, h_faces);
     ref_.logic = at(o_logic, h_logic);

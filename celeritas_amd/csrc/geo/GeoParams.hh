@@ -66,11 +66,10 @@ class GeoParams
 
     // Host copies (also exported for the test harness)
     std::vector<SurfaceRecord> h_surfaces;
-    std::vector<std::uint32_t> h_surf_offset;
-    std::vector<double> h_surf_data;
+    std::vector<double> h_planes;
     std::vector<SurfaceRecord> h_faces;
     std::vector<VolumeRecord> h_volumes;
-    std::vector<std::int32_t> h_logic;
+    std::vector<std::int8_t> h_logic;
     std::vector<double> h_bbox;
     std::vector<std::uint32_t> h_conn_begin;
     std::vector<std::uint32_t> h_conn_size;

@@ -146,6 +146,13 @@ struct GeoTrack
 //---------------------------------------------------------------------------//
 // SURFACE EVALUATION
 //---------------------------------------------------------------------------//
+//! Normal and displacement of a general plane
+CELER_FORCEINLINE_FUNCTION double const*
+plane_of(GeoParamsRef const& p, SurfaceRecord const& s)
+{
+    return p.planes + 4 * static_cast<std::uint32_t>(s.coeff);
+}
+
 //! Quadric value whose sign gives the sense
 CELER_FUNCTION double
 eval_surface(GeoParamsRef const& p, SurfaceRecord const& s, double const* x)
@@ -153,7 +160,7 @@ eval_surface(GeoParamsRef const& p, SurfaceRecord const& s, double const* x)
     double const c = s.coeff;
     if (s.type == SurfaceType::p)
     {
-        double const* d = p.surf_data + p.surf_offset[s.id];
+        double const* d = plane_of(p, s);
         return d[0] * x[0] + d[1] * x[1] + d[2] * x[2] - d[3];
     }
     switch (s.type)
@@ -250,7 +257,7 @@ CELER_FUNCTION void calc_intersections(GeoParamsRef const& p,
     }
     if (t == SurfaceType::p)
     {
-        double const* d = p.surf_data + p.surf_offset[s.id];
+        double const* d = plane_of(p, s);
         double const n_dir = d[0] * u[0] + d[1] * u[1] + d[2] * u[2];
         if (!on && n_dir != 0)
         {
@@ -303,7 +310,7 @@ CELER_FUNCTION void calc_normal(GeoParamsRef const& p,
     }
     if (t == SurfaceType::p)
     {
-        double const* d = p.surf_data + p.surf_offset[s.id];
+        double const* d = plane_of(p, s);
         n[0] = d[0];
         n[1] = d[1];
         n[2] = d[2];
@@ -412,7 +419,7 @@ CELER_FUNCTION bool
 eval_logic(GeoParamsRef const& p, std::uint32_t vol, std::uint32_t senses)
 {
     VolumeRecord const record = p.volumes[vol];
-    std::int32_t const* lg = p.logic + record.logic_begin;
+    std::int8_t const* lg = p.logic + record.logic_begin;
     int const n = record.logic_size;
     std::uint64_t stack = 0;
     for (int i = 0; i < n; ++i)

@@ -55,11 +55,9 @@ hipError_t CELER_PREC_FN(launch_along_step_charged)(CoreParamsRef const& p,
                                      hipStream_t st)
 {
     // Physics and geometry tables in LDS where both fit, else the physics
-    unsigned int lds = staged_both_bytes(p);
-    Staging const staging = lds ? Staging::both
-                                : (staged_table_bytes(p) ? Staging::physics : Staging::none);
-    if (staging == Staging::physics)
-        lds = staged_table_bytes(p);
+    Staging const staging = charged_staging(p);
+    unsigned int const lds = staging == Staging::both ? staged_both_bytes(p)
+                                                      : staged_table_bytes(p);
     auto pick = [staging](auto both, auto physics, auto none) {
         return staging == Staging::both ? both : staging == Staging::physics ? physics : none;
     };

@@ -13,9 +13,9 @@
 //! dynamic LDS copies the regions it reads once per workgroup and continues
 //! with a params view whose table pointers are rebased into LDS, so the
 //! chains of dependent table reads of a track (particle -> process -> grid
-//! header -> values; volume -> faces) are served
-//! from LDS instead of L2. The data are the same bytes, so results are
-//! bit-identical to the unstaged path.
+//! header -> values; volume -> faces) are served from LDS instead of L2. The
+//! data are the same bytes, so results are bit-identical to the unstaged
+//! path. StagingRules.hh says which regions a launch stages.
 //---------------------------------------------------------------------------//
 #pragma once
 
@@ -25,59 +25,12 @@
 
 #include "corecel/WaveOps.hh"
 #include "CoreData.hh"
+#include "StagingRules.hh"
 #include "StepExecutors.hh"
 
 namespace celeritas_amd
 {
 //---------------------------------------------------------------------------//
-//! Largest region staged: above it a kernel reads the tables in place (at
-//! 32 KiB five 256-thread workgroups still fit a CU's LDS)
-inline constexpr unsigned int max_staged_table_bytes = 32 * 1024;
-//! Largest physics and geometry regions staged together (three 256-thread
-//! workgroups per CU, the register limit of the kernel that stages both)
-inline constexpr unsigned int max_staged_both_bytes = 52 * 1024;
-
-//! Dynamic LDS bytes of a launch staging the physics tables (0: the tables
-//! stay in HBM)
-inline unsigned int staged_table_bytes(CoreParamsRef const& p)
-{
-    unsigned int const n = p.phys.hot_bytes;
-    return (n > 0 && n <= max_staged_table_bytes) ? n : 0;
-}
-
-//! Dynamic LDS bytes of a launch staging the tables that finding distances
-//! reads
-inline unsigned int staged_geo_bytes(CoreParamsRef const& p)
-{
-    unsigned int const n = p.geo.track_bytes;
-    return (n > 0 && n <= max_staged_table_bytes) ? n : 0;
-}
-
-//! Dynamic LDS bytes of a launch staging all geometry tables
-inline unsigned int staged_crossing_bytes(CoreParamsRef const& p)
-{
-    unsigned int const n = p.geo.hot_bytes;
-    return (n > 0 && n <= max_staged_table_bytes) ? n : 0;
-}
-
-//! Dynamic LDS bytes of a launch staging physics and distances (physics first)
-inline unsigned int staged_both_bytes(CoreParamsRef const& p)
-{
-    unsigned int const a = staged_table_bytes(p);
-    unsigned int const b = staged_geo_bytes(p);
-    return (a > 0 && b > 0 && a + b <= max_staged_both_bytes) ? a + b : 0;
-}
-
-//! What a launch stages in LDS
-enum class Staging
-{
-    none,
-    physics,
-    geometry,  //!< what finding distances reads
-    crossing,  //!< all of the geometry
-    both,  //!< physics and geometry
-};
-
 /*!
  * Whether any thread of this workgroup maps to a slot.
  *
@@ -157,8 +110,7 @@ __device__ __forceinline__ void rebase_geometry(GeoParamsRef* r, char* to)
     GeoParamsRef const g = *r;
     char const* from = g.hot_base;
     r->surfaces = rebase(g.surfaces, from, to);
-    r->surf_offset = rebase(g.surf_offset, from, to);
-    r->surf_data = rebase(g.surf_data, from, to);
+    r->planes = rebase(g.planes, from, to);
     r->volumes = rebase(g.volumes, from, to);
     r->faces = rebase(g.faces, from, to);
     r->logic = rebase(g.logic, from, to);
@@ -182,11 +134,11 @@ __device__ __forceinline__ void rebase_crossing(GeoParamsRef* r, char* to)
  * first, then the geometry region).
  *
  * Every thread of the workgroup must call this before any of them returns
- * (it contains a workgroup barrier). The launcher gives the kernel the
- * LDS its staging needs (staged_table_bytes, staged_geo_bytes,
- * staged_crossing_bytes, staged_both_bytes) and instantiates it with that staging only when the
- * regions fit: the table pointers then derive from the LDS array alone,
- * so the compiler reads them with LDS instructions and 32-bit addresses.
+ * (it contains a workgroup barrier). The launcher gives the kernel the LDS
+ * its staging needs (StagingRules.hh) and instantiates it with that staging
+ * only when the regions fit: the table pointers then derive from the LDS
+ * array alone, so the compiler reads them with LDS instructions and 32-bit
+ * addresses.
  */
 template<Staging S>
 __device__ __forceinline__ CoreParamsRef stage(CoreParamsRef const& params, void* lds)
