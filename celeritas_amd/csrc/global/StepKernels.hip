@@ -121,9 +121,11 @@ __global__ void __launch_bounds__(block_size)
 // INTERACTIONS
 //---------------------------------------------------------------------------//
 //! One instantiation per model class: each launch carries only the
-//! registers of its own sampler
+//! registers of its own sampler, and at least three waves per SIMD like the
+//! launch of all models (combined bremsstrahlung 179 -> 167 registers; a
+//! TestEm3 step's 56 us of it wait for memory either way)
 template<ModelClass M>
-__global__ void __launch_bounds__(block_size)
+__global__ void __launch_bounds__(block_size, 3)
     interaction_kernel(CoreParamsRef const params,
                        CoreStateRef const state,
                        std::uint8_t const action,

@@ -45,6 +45,23 @@ def test_step_kernels_recorded(amd):
             assert a["local_mem"] == 0, name  # no register spills on the hot path
 
 
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_models_in_their_own_launches(amd, precision):
+    """Three waves per SIMD, as in the launch of all models, and no spills."""
+    physics = amd_pkg.generate_physics(wl.testem3_physics_spec())
+    prob = wl.testem3_problem(physics=physics, init_capacity=1 << 16, max_events=64,
+                              track_order="reindex_both_action", precision=precision)
+    stepper = amd.Stepper(amd.CoreParams(dict(prob, fuse_interactions=False)), 4096)
+    stepper(wl.testem3_primaries(4, emin=1e3, emax=2e3, seed=3))
+    suffix = "-mixed" if precision == "mixed" else ""
+    kernels = [a for a in amd_pkg.kernel_attributes()
+               if a["name"].startswith("interaction-")
+               and a["name"].endswith("-mixed") == bool(suffix)]
+    assert "interaction-combined_brem" + suffix in {a["name"] for a in kernels}
+    for a in kernels:
+        assert a["waves_per_simd"] >= 3 and a["local_mem"] == 0, a["name"]
+
+
 def test_kernel_timing(amd):
     """Launches carry dispatch start/stop events only while timing is on."""
     physics = amd_pkg.generate_physics(wl.testem3_physics_spec())
