@@ -524,9 +524,9 @@ PERSISTENT_FIELDS = [
     ("particle.particle_id", 1, False), ("particle.energy", 8, True),
     ("geo.pos", 24, True), ("geo.dir", 24, True), ("geo.volume", 4, True),
     ("geo.surface", 4, True), ("geo.sense", 1, True), ("geo.boundary", 1, True),
-    ("geo.failed", 1, False), ("geo.next_step", 8, True), ("geo.next_surface", 4, True),
-    ("geo.next_sense", 1, True), ("phys.interaction_mfp", 8, True),
-    ("phys.msc_range", 24, True), ("rng.xorwow", 24, True),
+    ("geo.failed", 1, False), ("geo.next_step", 8, True),
+    ("phys.interaction_mfp", 8, True), ("phys.msc_range", 24, True),
+    ("rng.xorwow", 24, True),
 ]
 #: Per new track: the secondary written to the stack and read back (40 B
 #: each way) and the initializer written and read (80 B each way)

@@ -179,8 +179,6 @@ struct GeoStateRef
     std::uint8_t* boundary{nullptr};  //!< BoundaryResult
     std::uint8_t* failed{nullptr};
     double* next_step{nullptr};
-    std::uint32_t* next_surface{nullptr};
-    std::uint8_t* next_sense{nullptr};
 };
 
 //---------------------------------------------------------------------------//

@@ -42,7 +42,8 @@ CELER_FORCEINLINE_FUNCTION int real_to_sense(double q)
 }
 
 //---------------------------------------------------------------------------//
-//! Track state held in registers by a kernel
+//! Track state held in registers by a kernel (the surface and sense of the
+//! next boundary do not outlive it and have no place in memory)
 struct GeoTrack
 {
     double pos[3];
@@ -101,8 +102,6 @@ struct GeoTrack
         this->store_turned(s, i);
         s.volume[i] = volume;
         s.failed[i] = failed;
-        s.next_surface[i] = next_surface;
-        s.next_sense[i] = next_sense;
     }
     /*!
      * What a move changes.

@@ -66,8 +66,6 @@ CoreState::CoreState(CoreParams const& params,
     add(&s.geo.boundary, n);
     add(&s.geo.failed, n);
     add(&s.geo.next_step, n);
-    add(&s.geo.next_surface, n);
-    add(&s.geo.next_sense, n);
     add(&s.phys.interaction_mfp, n);
     add(&s.phys.macro_xs, n);
     add(&s.phys.per_process_xs, n * max_processes);
@@ -180,7 +178,6 @@ void CoreState::reset()
                                       hipMemcpyHostToDevice, stream_));
     }
     CELER_HIP_CALL(launch_fill_u32(s.geo.surface, s.size, invalid_id, stream_));
-    CELER_HIP_CALL(launch_fill_u32(s.geo.next_surface, s.size, invalid_id, stream_));
     CELER_HIP_CALL(launch_fill_u32(s.sim.track_id, s.size, invalid_id, stream_));
     CELER_HIP_CALL(launch_fill_u32(s.sim.parent_id, s.size, invalid_id, stream_));
     CELER_HIP_CALL(launch_fill_u32(s.sim.event_id, s.size, invalid_id, stream_));

@@ -753,7 +753,6 @@ __global__ void __launch_bounds__(block_size)
                     state.geo.dir[k][slot] = ti.dir[k];
                 state.geo.failed[slot] = 0;
                 state.geo.next_step[slot] = 0;
-                state.geo.next_surface[slot] = invalid_id;
                 reset_physics(state.phys, slot);
                 to_slot = false;
             }

@@ -124,7 +124,7 @@ struct HostState
     HostState(size_type n, std::uint32_t num_proc)
     {
         // Offsets into three pools, filled in the order of the fields below
-        size_type const nu32 = 16 + 6, nf64 = 17 + num_proc, nu8 = 12;
+        size_type const nu32 = 15 + 6, nf64 = 17 + num_proc, nu8 = 11;
         u32.assign(std::size_t(n) * nu32, 0);
         f64.assign(std::size_t(n) * nf64, 0);
         u8.assign(std::size_t(n) * nu8, 0);
@@ -160,8 +160,6 @@ struct HostState
         s.geo.boundary = B();
         s.geo.failed = B();
         s.geo.next_step = F();
-        s.geo.next_surface = U();
-        s.geo.next_sense = B();
         s.phys.interaction_mfp = F();
         s.phys.macro_xs = F();
         s.phys.per_process_xs = pf;
