@@ -17,7 +17,7 @@ import numpy as np
 import pytest
 
 import celeritas_amd as amd_pkg
-from celeritas_amd import serving
+from celeritas_amd import serving, user
 from celeritas_amd import workloads as wl
 
 pytestmark = pytest.mark.gpu
@@ -73,7 +73,7 @@ def test_events_overlap(amd, params):
 def test_tally_of_more_events_than_bins(amd, params, slots):
     """Events 1,024 apart share a bin of the workgroups' sums (those that
     come second add to memory directly), and the last chunk of slots is
-    partly filled: no deposit and no track is lost."""
+    partly filled: every event completes, and no deposit is lost."""
     server = serving.Server(params, slots)
     events = wl.served_events(1100, seed=17, nmin=1, nmax=2, emin=100.0, emax=200.0)
     r = server.run(events, np.zeros(len(events)), max_steps=200_000)
@@ -83,6 +83,47 @@ def test_tally_of_more_events_than_bins(amd, params, slots):
     if slots >= 1 << 14:
         # All fit at once, so such pairs were in flight together
         assert np.any(r["admit"][1024:] <= r["done"][:76])
+
+
+@pytest.mark.parametrize("slots", [1000, (1 << 14) + 123])
+def test_track_ids_of_more_events_than_bins(amd, slots):
+    """Every track of an event has an ID of its own, and the event's IDs are
+    those below its counter, also where events share a bin of the workgroups'
+    sums and in the last, partly filled chunk of slots: in the slots and the
+    queue of a run stopped on its way, and over a whole run by its tracks'
+    first steps."""
+    problem = wl.testem3_problem(physics=amd_pkg.generate_physics(wl.testem3_physics_spec()),
+                                 init_capacity=1 << 20, max_events=1 << 12,
+                                 track_order="reindex_both_action")
+    events = wl.served_events(1100, seed=17, nmin=1, nmax=2, emin=100.0, emax=200.0)
+    zeros = np.zeros(len(events))
+
+    server = serving.Server(amd.CoreParams(problem), slots)
+    with pytest.raises(amd_pkg.CeleritasError, match="exceeded 24 steps"):
+        server.run(events, zeros, max_steps=24)
+    state = server.state
+    queue = state.get("initializers", state.counters()["num_initializers"])
+    occupied = state.get("status") != amd_pkg.TRACK_STATUS["inactive"]
+    event = np.concatenate([state.get("event_id")[occupied], queue["event_id"]])
+    track = np.concatenate([state.get("track_id")[occupied], queue["track_id"]])
+    counters = state.get("track_counters", len(events))
+    assert occupied.sum() > 500 and event.max() >= 1024
+    assert counters.sum() > len(track)
+    assert len(np.unique(np.stack([event, track]), axis=1).T) == len(track)
+    assert np.all(track < counters[event])
+
+    params = amd.CoreParams(problem)
+    hits = user.StepCollector(params, user.StepSelection(event_id=True, track_step_count=True),
+                              hit_capacity=1 << 22)
+    server = serving.Server(params, slots)
+    server.run(events, zeros, max_steps=200_000)
+    h = hits.read()
+    assert h["overflow_steps"] == 0
+    first = h["track_step_count"] == 1
+    counters = server.state.get("track_counters", len(events))
+    pairs = np.stack([h["event_id"][first], h["track_id"][first]])
+    assert np.all(pairs[1] < counters[pairs[0]])
+    assert len(np.unique(pairs, axis=1).T) == first.sum() == counters.sum()
 
 
 def test_device_admission_in_order_within_limit(amd, params):
