@@ -31,10 +31,19 @@ def test_overflow_in_a_batch_of_steps(amd, graph):
             stepper.run_steps(32)
     c = stepper.state.counters()
     assert c["num_initializers"] > capacity
-    # Slots still hold real tracks only: no more than there are, in the world
+    # The batch's last steps started no tracks, though slots were free
+    assert c["num_new_tracks"] == 0 and c["num_vacancies"] > 0
+    # Slots still hold real tracks only: each its own, with an ID that its
+    # event has given out (initializers that were never written are zero: the
+    # first track of event 0, again and again)
     status = stepper.state.get("status")
-    assert c["num_alive"] <= slots and np.all(status <= 4)
+    occupied = status != amd_pkg.TRACK_STATUS["inactive"]
+    assert c["num_alive"] <= slots and np.all(status <= 4) and occupied.sum() > 1
     assert np.all(stepper.state.get("energy") <= 1e4)
+    event = stepper.state.get("event_id")[occupied]
+    track = stepper.state.get("track_id")[occupied]
+    assert len(np.unique(np.stack([event, track]), axis=1).T) == occupied.sum()
+    assert np.all(track < stepper.state.get("track_counters", 512)[event])
 
     # The state is whole again after a reset
     stepper.state.reset()
