@@ -398,12 +398,13 @@ struct TallyBins
 /*!
  * Add to an event's count of live tracks and initializers.
  *
- * A track only changes its own event's count by -1 (death without
- * secondaries) or more, and every other live track or initializer of the
- * event is still counted, so the update that takes the count to zero is the
- * event's completion. The same holds for the sums of disjoint sets of
- * tracks, of which those that sum to zero are left out: a partial sum is
- * zero only if every track of the event is in it and none has a successor.
+ * Each of the event's tracks changes the count by -1 (death without
+ * secondaries) or more. So it reaches zero only once every track has been
+ * added, each with -1, and no initializer waits: the update that takes it
+ * there is the event's completion, in whatever order the updates come and
+ * also where they are sums over disjoint sets of tracks. A sum of zero can
+ * be left out: its set is empty, or holds a track that did not contribute
+ * -1, and then the event goes on.
  */
 __device__ __forceinline__ void
 add_live(CoreStateRef const& state, std::uint32_t event, int delta)
