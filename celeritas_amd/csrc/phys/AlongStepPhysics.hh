@@ -276,21 +276,6 @@ CELER_FUNCTION double calc_eloss(PhysicsParamsRef const& p,
     return eloss;
 }
 
-template<class Engine>
-CELER_FUNCTION double calc_eloss(PhysicsParamsRef const& p,
-                                 ParticlePhysics const& part,
-                                 std::uint32_t pid,
-                                 std::uint32_t mat,
-                                 double energy,
-                                 double range,
-                                 double step,
-                                 bool apply_cut,
-                                 Engine& rng)
-{
-    phys::GridPoint gp(energy);
-    return calc_eloss(p, part, pid, mat, gp, range, step, apply_cut, rng);
-}
-
 //---------------------------------------------------------------------------//
 // URBAN MULTIPLE SCATTERING
 //---------------------------------------------------------------------------//

@@ -102,13 +102,6 @@ calc_grid(XsGrid const& g, double const* __restrict__ reals, GridPoint& gp)
     return result;
 }
 
-CELER_FUNCTION double
-calc_grid(XsGrid const& g, double const* __restrict__ reals, double energy)
-{
-    GridPoint gp(energy);
-    return calc_grid(g, reals, gp);
-}
-
 inline constexpr double r_electron = 2.8179403262e-13;  //!< [cm]
 
 //! Heitler e+ annihilation macroscopic cross section [1/cm]
@@ -185,13 +178,6 @@ calc_range(XsGrid const& g, double const* __restrict__ reals, GridPoint& gp)
     std::uint32_t const i = gp.lower;
     double const slope = ((-v[i]) + v[i + 1]) / ((-gp.lower_e) + gp.upper_e);
     return std::fma(slope, (-gp.lower_e) + gp.energy, v[i]);
-}
-
-CELER_FUNCTION double
-calc_range(XsGrid const& g, double const* __restrict__ reals, double energy)
-{
-    GridPoint gp(energy);
-    return calc_range(g, reals, gp);
 }
 
 /*!

@@ -118,7 +118,8 @@ int main(int argc, char** argv)
         // Along-step physics of charged particles
         if (part.eloss_process < 0) continue;
         double const energy = logu(1e-3, 1e5);
-        double const range = phys::calc_range(p.grids[part.range_grid + mat], p.grid_reals, energy);
+        phys::GridPoint gp(energy);
+        double const range = phys::calc_range(p.grids[part.range_grid + mat], p.grid_reals, gp);
         bool const lepton = pid == p.electron_id || pid == p.positron_id;
         double step = range * logu(1e-6, 1.0);
         double safety = U(gen) < 0.2 ? 0.0 : logu(1e-7, 5.0);
@@ -159,7 +160,7 @@ int main(int argc, char** argv)
                     if (bad) { ++nbad; if (nbad < 20) std::printf("BAD MSC: %s -> true %.9g geom %.9g |dir|^2 %.9g action %d\n", g_case, true_path, geom_path, n, res.action); }
                 }
             }
-            double dep = alongstep::calc_eloss(p, part, pid, mat, energy, range, true_path, U(gen) < 0.5, rng);
+            double dep = alongstep::calc_eloss(p, part, pid, mat, gp, range, true_path, U(gen) < 0.5, rng);
             if (nanmode >= 0.3 && !(dep >= 0 && dep <= energy)) { ++nbad; if (nbad < 20) std::printf("BAD ELOSS: %s -> %.9g\n", g_case, dep); }
         }
         catch (Limit const&) { ++fails; std::printf("LOOP: %s\n", g_case); }
