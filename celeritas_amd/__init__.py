@@ -575,6 +575,20 @@ def verify_field_propagate(params: CoreParams, tracks, steps,
     return out
 
 
+def verify_elementary(x) -> tuple[np.ndarray, np.ndarray, np.ndarray]:
+    """Logarithm, sine and cosine of ``x`` by the step kernels' own FP64
+    functions on the device."""
+    f = _load().celer_verify_elementary
+    f.argtypes = [ctypes.c_void_p, ctypes.c_uint32, ctypes.c_void_p, ctypes.c_void_p]
+    f.restype = ctypes.c_int
+    x = np.ascontiguousarray(x, np.float64).ravel()
+    out = np.zeros((3, len(x)))
+    rc = f(x.ctypes.data, len(x), out.ctypes.data, None)
+    if rc != 0:
+        raise CeleritasError(f"celer_verify_elementary failed with HIP error {rc}")
+    return out[0], out[1], out[2]
+
+
 def verify_geo_locate(params: CoreParams, points) -> np.ndarray:
     """Volume of each point (rows of pos[3], dir[3]) as found by track
     initialization on the device; 0xffffffff where it fails."""

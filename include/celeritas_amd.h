@@ -590,6 +590,13 @@ int celer_verify_field_propagate(const void* params_ref,
                                  void* stream);
 
 /*---------------------------------------------------------------------------*
+ * VERIFICATION: the FP64 logarithm, sine and cosine of the step kernels, on
+ * the device. Writes 3 n doubles: the logarithms of the n arguments, their
+ * sines and their cosines (these for angles of up to 2^20 radians).
+ *---------------------------------------------------------------------------*/
+int celer_verify_elementary(const double* x, uint32_t n, double* out, void* stream);
+
+/*---------------------------------------------------------------------------*
  * VERIFICATION: point location as in track initialization
  * (orange/univ/SimpleUnitTracker.hh:161-190, candidates from the BIH of
  * orange/detail/BIHTraverser.hh). Each of n points is 6 doubles (pos [cm],

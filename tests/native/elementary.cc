@@ -26,8 +26,9 @@ int main(int argc, char** argv)
     {
         // A positive range over decades is sampled by its logarithm
         double const u = uniform(rng);
-        double const x = (lo > 0 && hi / lo > 1e3) ? lo * std::pow(hi / lo, u)
-                                                   : lo + (hi - lo) * u;
+        long double const ratio = static_cast<long double>(hi) / lo;
+        double const x = (lo > 0 && ratio > 1e3) ? static_cast<double>(lo * powl(ratio, u))
+                                                 : lo + (hi - lo) * u;
         double s, c, got;
         long double want;
         if (fn == "log")
@@ -46,7 +47,7 @@ int main(int argc, char** argv)
         int e;
         std::frexp(static_cast<double>(want), &e);
         double const err = std::fabs(static_cast<double>((got - want) / ldexpl(1.0L, e - 53)));
-        if (err > worst)
+        if (!(err <= worst))
         {
             worst = err;
             at = x;
