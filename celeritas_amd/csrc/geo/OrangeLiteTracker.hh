@@ -838,31 +838,36 @@ CELER_FUNCTION void cross_boundary(GeoParamsRef const& p, GeoTrack& g)
     g.volume = found;
 }
 
+//! Whether two directions at a point of a surface point to different sides
+CELER_FORCEINLINE_FUNCTION bool changes_side(GeoParamsRef const& p,
+                                             std::uint32_t surface,
+                                             double const* x,
+                                             double const* olddir,
+                                             double const* newdir)
+{
+    double n[3];
+    calc_normal(p, p.surfaces[surface], x, n);
+    double const dn_new = n[0] * newdir[0] + n[1] * newdir[1] + n[2] * newdir[2];
+    double const dn_old = n[0] * olddir[0] + n[1] * olddir[1] + n[2] * olddir[2];
+    return (dn_new >= 0) != (dn_old >= 0);
+}
+
 /*!
  * Change direction; on a boundary this may make the crossing reentrant.
  */
 CELER_FUNCTION void
 set_dir(GeoParamsRef const& p, GeoTrack& g, double const* newdir)
 {
-    if (g.is_on_boundary())
-    {
-        double n[3];
-        calc_normal(p, p.surfaces[g.surface], g.pos, n);
-        double const dn_new = n[0] * newdir[0] + n[1] * newdir[1]
-                              + n[2] * newdir[2];
-        double const dn_old = n[0] * g.dir[0] + n[1] * g.dir[1]
-                              + n[2] * g.dir[2];
-        if ((dn_new >= 0) != (dn_old >= 0))
-            g.boundary ^= 1u;
-    }
+    if (g.is_on_boundary() && changes_side(p, g.surface, g.pos, g.dir, newdir))
+        g.boundary ^= 1u;
     for (int k = 0; k < 3; ++k)
         g.dir[k] = newdir[k];
     g.clear_next();
 }
 
 /*!
- * Change the direction of the track in a slot; its position and old
- * direction are read only on a boundary.
+ * The same for the track in a slot; its position and old direction are read
+ * only on a boundary.
  */
 CELER_FUNCTION void set_dir(GeoParamsRef const& p,
                             GeoStateRef const& s,
@@ -872,15 +877,13 @@ CELER_FUNCTION void set_dir(GeoParamsRef const& p,
     std::uint32_t const surface = s.surface[i];
     if (surface != invalid_id)
     {
-        double x[3], n[3];
+        double x[3], dir[3];
         for (int k = 0; k < 3; ++k)
+        {
             x[k] = s.pos[k][i];
-        calc_normal(p, p.surfaces[surface], x, n);
-        double const dn_new = n[0] * newdir[0] + n[1] * newdir[1]
-                              + n[2] * newdir[2];
-        double const dn_old = n[0] * s.dir[0][i] + n[1] * s.dir[1][i]
-                              + n[2] * s.dir[2][i];
-        if ((dn_new >= 0) != (dn_old >= 0))
+            dir[k] = s.dir[k][i];
+        }
+        if (changes_side(p, surface, x, dir, newdir))
             s.boundary[i] ^= 1u;
     }
     for (int k = 0; k < 3; ++k)
