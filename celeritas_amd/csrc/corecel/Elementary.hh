@@ -9,14 +9,23 @@
 //! issue. The library carries a logarithm as a pair of doubles from start to
 //! end (98 vector instructions; 72 here) and reduces any angle up to the
 //! largest double, once for the sine and once for the cosine (260 for both;
-//! 70 here). Largest errors on the device, in units of the last place, of 4
-//! million values a range: logarithm of (0, 1) 0.594 (library 0.641), of
-//! 10^-300 to 10^300 0.545 (0.610); sine and cosine of -10 to 10 0.724
-//! (0.783). Full TestEm3 transport 840 -> 825 ms,
-//! graph replay of 333 primaries 48.8 -> 47.5 ms.
+//! 70 here). Full TestEm3 transport 840 -> 825 ms, graph replay of 333
+//! primaries 48.8 -> 47.5 ms.
 //!
+//! Largest errors on the device in units of the last place, of eight million
+//! values a range (library in parentheses): logarithm of (0, 1) 0.599
+//! (0.641), of 0.5 to 2 0.602 (0.637), of 10^-300 to 10^300 0.538 (0.607);
+//! sine and cosine of -10 to 10 0.727 (0.779). The mean errors are smaller,
+//! too. One part is not: just beside sqrt(1/2) and sqrt(2), where the
+//! reduction folds, the logarithm's largest error is 0.611 (0.591 in 1.4142
+//! to 1.4143) at a mean of 0.251 (0.254).
+//!
+//! The logarithm's sum has the form that K. C. Ng published with Sun's
+//! freely distributable math library (1993), here with the rounding errors
+//! of its large terms; the angle's reduction is Cody and Waite's.
 //! Coefficients are interpolations in Chebyshev nodes of the series, taken
-//! with 60 digits. The same functions compile for the host.
+//! with 60 digits. The same functions compile for the host; angles above
+//! 2^20 radians are out of their range (the kernels' stay below 10).
 //---------------------------------------------------------------------------//
 #pragma once
 

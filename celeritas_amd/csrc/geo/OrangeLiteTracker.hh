@@ -110,7 +110,7 @@ struct GeoTrack
      * for one or two tracks, so every field that a kernel only wrote back
      * cost several times its bytes: the stores hold the fields that change
      * (2^20 slots: interactions 99 -> 92, boundary 80 -> 71, both along-step
-     * kernels together 245 -> 240 us a step; neutral along-step 110 -> 91
+     * kernels together 245 -> 240 us a step; neutral along-step 110 -> 95
      * registers, five waves per SIMD).
      */
     CELER_FORCEINLINE_FUNCTION void store_moved(GeoStateRef const& s,

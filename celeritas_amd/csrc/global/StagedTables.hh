@@ -63,8 +63,8 @@ __device__ __forceinline__ T const* rebase(T const* p, char const* from, char* t
  * Copy a 16-byte-aligned region into LDS (no barrier).
  *
  * Each thread has a batch of loads in flight before it writes any: a loop
- * of load and write waited for the memory once per 4 KiB, 13 times for the
- * tables of the charged along-step (2^20 slots: pre-step 67 -> 61 us a step;
+ * of load and write waited for the memory once per 4 KiB, 12 times for the
+ * 46 KB of the charged along-step (2^20 slots: pre-step 67 -> 61 us a step;
  * full TestEm3 transport 885 -> 874 ms).
  */
 __device__ __forceinline__ void copy_region(char const* from, unsigned int n, char* to)

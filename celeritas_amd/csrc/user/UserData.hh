@@ -119,6 +119,8 @@ struct StepHitCounters
 struct StepHitColumns
 {
     static constexpr unsigned int max_columns = 20;
+    // Detector and track, and one for each property that can be selected
+    static_assert(2 + sizeof(StepSelection) <= max_columns, "columns of a hit");
     struct Column
     {
         std::uint32_t const* data;
