@@ -61,16 +61,19 @@ BYTES_PER_UNIT = {
     # range written
     "pre-step": (93, 1, "pre_step"),
     # geometry state (position, direction, volume, surface, sense, boundary
-    # flags, next-step cache: 72 B read, 68 B written), RNG state (24 + 24),
-    # MSC range state (24 + 24), step, actions, energy, time, range, MFP,
-    # macro XS, deposition, step count (184 B read, 161 B written in all)
-    "along-step-general-linear": (345, 2, "along_charged"),
+    # flag: 58 B read; without the volume and with the next step 62 B
+    # written), RNG state (24 + 24), MSC range state (24 + 24), step,
+    # actions, energy, time, range, MFP, macro XS, deposition, step count
+    # (170 B read, 155 B written in all)
+    "along-step-general-linear": (325, 2, "along_charged"),
     # the same plus the looping-step counter
-    "along-step-uniform-msc": (353, 2, "along_charged"),
-    # geometry state, step, actions, time, MFP, macro XS, energy, steps
-    "along-step-neutral": (216, 2, "along_neutral"),
-    # geometry state read and written, status, action
-    "geo-boundary": (142, 2, "boundary"),
+    "along-step-uniform-msc": (333, 2, "along_charged"),
+    # geometry state (58 B read; position, surface, sense and next step
+    # written: 37 B), step, actions, time, MFP, macro XS, energy, steps
+    "along-step-neutral": (171, 2, "along_neutral"),
+    # geometry state read, volume, sense and boundary flag written, status,
+    # action
+    "geo-boundary": (66, 2, "boundary"),
 }
 
 
@@ -516,7 +519,8 @@ def sorted_launch(label, track_order):
 #: geo/GeoData.hh, phys/PhysicsData.hh, random/XorwowEngine.hh). Fields a
 #: step computes and consumes itself (cross sections, step length and
 #: actions, deposition, secondary span, element) are not persistent: in a
-#: step fused into one kernel they would stay in registers.
+#: step fused into one kernel they would stay in registers. Nor is the next
+#: step to a boundary, which every kernel finds for itself.
 PERSISTENT_FIELDS = [
     # (field, bytes, written back by a step)
     ("sim.track_id", 4, False), ("sim.parent_id", 4, False), ("sim.event_id", 4, False),
@@ -524,9 +528,8 @@ PERSISTENT_FIELDS = [
     ("particle.particle_id", 1, False), ("particle.energy", 8, True),
     ("geo.pos", 24, True), ("geo.dir", 24, True), ("geo.volume", 4, True),
     ("geo.surface", 4, True), ("geo.sense", 1, True), ("geo.boundary", 1, True),
-    ("geo.failed", 1, False), ("geo.next_step", 8, True),
-    ("phys.interaction_mfp", 8, True), ("phys.msc_range", 24, True),
-    ("rng.xorwow", 24, True),
+    ("geo.failed", 1, False), ("phys.interaction_mfp", 8, True),
+    ("phys.msc_range", 24, True), ("rng.xorwow", 24, True),
 ]
 #: Per new track: the secondary written to the stack and read back (40 B
 #: each way) and the initializer written and read (80 B each way)
